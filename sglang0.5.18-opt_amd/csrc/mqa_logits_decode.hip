@@ -40,6 +40,8 @@
 //    bins a word; a CTA's tokens per row stay below 2^16) flushed once per CTA with one global
 //    atomic per nonzero bin; mqa_hist_init_kernel seeds the zero bin / zero count with the row
 //    length (mqa_hist.cu:278-304) and every CTA subtracts its nonzero tokens.
+#include <algorithm>
+
 #include "dsa_common.h"
 
 namespace dsa {
@@ -118,7 +120,7 @@ struct DecodeArgs {
   int32_t* zero_ws;   // non-null: the paired top-k's workspace, whose counters are zeroed here
   int64_t batch;
   int nt_logits;      // logits stored nontemporally (a logits block larger than the L2s hold)
-  int slice_pages;    // > 0: slice-major assignment (assign_slices) with slices of this many pages
+  int slice_pages;    // > 0: slice-major assignment with slices of this many pages
 };
 
 __device__ __forceinline__ int clamp_len(int l, int width) { return l < 0 ? 0 : (l > width ? width : l); }
@@ -194,61 +196,16 @@ __device__ void assign_cta(const DecodeArgs& a, int (&s_w)[2][NT / kWave], int* 
   }
 }
 
-// Slice-major assignment (the prefill launches): the K pages of every group are cut into slices of
-// SL = a.slice_pages pages, and CTA c takes the c-th (slice, group) pair in slice-then-group
-// order, so the CTAs resident at one time -- consecutive blockIdx, spread over the 8 XCDs by
-// blockIdx % 8 -- work on the same slice of K for different row groups: each XCD's L2 then holds
-// one slice (SL * 8448 B) that all of its CTAs read, where the group-major balanced grid has every
-// XCD's resident CTAs spread over the whole K range (a prefill's 10-20 MB of K misses the L2s).
-// s_assign = {group (-1: none), slice, the group's pages}.  Ends before a barrier (the caller's).
-constexpr int kMaxSlices = 64;  // slices a group may have (the host sizes SL for it)
+// Slice-major assignment (the prefill launches): the K pages are cut into slices of a.slice_pages
+// pages and CTA c takes slice c / n_groups of group c % n_groups, so the CTAs resident at one time --
+// consecutive blockIdx, spread over the 8 XCDs by blockIdx % 8 -- work on the same slice of K for
+// different row groups: each XCD's L2 then holds one slice that all of its CTAs read, where the
+// group-major balanced grid has every XCD's resident CTAs spread over the whole K range (a prefill's
+// 10-20 MB of K misses the L2s).  A pair past its group's pages leaves at once.  The host sizes the
+// slices (slice_count); the lengths are read for the CTA's own group only (ranking the non-empty
+// pairs first read every group's twice, behind three barriers, and packed a causal launch no better).
 
-template <int NT>
-__device__ void assign_slices(const DecodeArgs& a, int (&s_w)[2][NT / kWave], int* s_nsl, int* s_assign) {
-  const int tid = threadIdx.x;
-  const int cta = blockIdx.x;
-  const int SL = a.slice_pages;
-  // s_nsl[n] = groups with n slices
-  for (int i = tid; i <= kMaxSlices; i += NT) s_nsl[i] = 0;
-  if (tid == 0) s_assign[0] = -1;
-  __syncthreads();
-  for (int g = tid; g < a.n_groups; g += NT) {
-    const int ns = (group_pages(a, g) + SL - 1) / SL;
-    atomicAdd(&s_nsl[ns < kMaxSlices ? ns : kMaxSlices], 1);
-  }
-  __syncthreads();
-  // this CTA's slice j: pairs of slice j are the groups with more than j slices
-  int j = 0, before = 0, in_j = 0;
-  for (; j < kMaxSlices; ++j) {
-    in_j = 0;
-    for (int n = j + 1; n <= kMaxSlices; ++n) in_j += s_nsl[n];
-    if (cta < before + in_j) break;
-    before += in_j;
-  }
-  if (j == kMaxSlices) return;  // block-uniform: no pair left for this CTA
-  const int rank = cta - before;  // the rank-th group (in group order) with more than j slices
-  int seen = 0;
-  for (int g0 = 0; g0 < a.n_groups; g0 += NT) {  // block-uniform
-    const int g = g0 + tid;
-    int pages = 0;
-    bool has = false;
-    if (g < a.n_groups) {
-      pages = group_pages(a, g);
-      has = (pages + SL - 1) / SL > j;
-    }
-    int total;
-    const int pre = block_excl_sum<NT>(has ? 1 : 0, total, s_w[(g0 / NT) & 1]);
-    if (has && seen + pre == rank) {
-      s_assign[0] = g;
-      s_assign[1] = j;
-      s_assign[2] = pages;
-    }
-    seen += total;
-    if (seen > rank) break;  // block-uniform
-  }
-}
-
-// The same for up to 64 groups, computed by every wave on its own (lane g holds group g): no
+// The balanced assignment for up to 64 groups, computed by every wave on its own (lane g holds group g): no
 // LDS and no barrier before the CTA's first block-table read.  Returns {group (-1: none), index
 // within the group's CTAs, their count}, wave-uniform.
 __device__ __forceinline__ int3 assign_cta_wave(const DecodeArgs& a) {
@@ -326,7 +283,6 @@ __global__ __launch_bounds__((Shape<R, kHist>::kThreads)) __attribute__((amdgpu_
   __shared__ int s_cnt[2 * R];
   __shared__ int s_w[2][NT / kWave];
   __shared__ int s_assign[3];  // group, index within the group's CTAs, the group's CTA count
-  __shared__ int s_nsl[kMask ? 1 : kMaxSlices + 1];  // slice-major assignment (prefill, no mask)
   __shared__ int s_bt[Sh::kMaxPages];
 
   const int tid = threadIdx.x;
@@ -335,17 +291,10 @@ __global__ __launch_bounds__((Shape<R, kHist>::kThreads)) __attribute__((amdgpu_
   const int cta = blockIdx.x;
 
   int grp, jc, nj;
-  int slice_begin = -1, slice_pages = 0;  // slice-major: the CTA's first page, its group's pages
   if (!kMask && a.slice_pages > 0) {  // block-uniform
-    if constexpr (!kMask) {
-      assign_slices<NT>(a, s_w, s_nsl, s_assign);
-      __syncthreads();
-      grp = s_assign[0];
-      jc = s_assign[1];
-      nj = 1;
-      slice_begin = jc * a.slice_pages;
-      slice_pages = s_assign[2];
-    }
+    jc = cta / a.n_groups;
+    grp = cta - jc * a.n_groups;
+    nj = 1;
   } else if (a.n_groups <= kWave) {  // block-uniform
     const int3 as = assign_cta_wave(a);
     grp = uniform(as.x);
@@ -390,9 +339,15 @@ __global__ __launch_bounds__((Shape<R, kHist>::kThreads)) __attribute__((amdgpu_
     hlim = h > kTopK ? h : 0;
   }
   const int pages = (max_len + kPage - 1) / kPage;
-  const int p_begin = slice_begin >= 0 ? slice_begin : static_cast<int>(static_cast<int64_t>(pages) * jc / nj);
-  const int p_end = slice_begin >= 0 ? min(slice_begin + a.slice_pages, slice_pages)
-                                     : static_cast<int>(static_cast<int64_t>(pages) * (jc + 1) / nj);
+  int p_begin, p_end;
+  if (!kMask && a.slice_pages > 0) {  // block-uniform
+    p_begin = jc * a.slice_pages;
+    p_end = min(p_begin + a.slice_pages, pages);
+    if (p_begin >= p_end) return;  // no page of this group in the slice
+  } else {
+    p_begin = static_cast<int>(static_cast<int64_t>(pages) * jc / nj);
+    p_end = static_cast<int>(static_cast<int64_t>(pages) * (jc + 1) / nj);
+  }
   const int n_local = p_end - p_begin;  // <= Sh::kMaxPages by the host's choice of target
   const int32_t* btr = a.bt + static_cast<int64_t>(group_row) * a.bt_stride + p_begin;
 
@@ -668,6 +623,30 @@ void shape_host(int R, bool hist, int& ctas_per_cu, int& max_pages) {
   }
 }
 
+// Pages of the slices a prefill launch of n_groups 8-row groups cuts its width_pages K pages into
+// (at most max_pages, the block-table stage).  A CU serves its CTAs at one rate whatever their number
+// from two up, and a CTA costs about one page beyond its own (q fragments, the first page's latency),
+// so a launch takes about rounds * (L + 1) pages, rounds = CTAs per CU rounded up; a lone CTA a CU
+// (two waves a SIMD) runs a third slower; and the CTAs, of unequal lengths when the rows are causal,
+// end spread over half a slice.  The L that makes this least is taken.  Against slices as long as the
+// block-table stage allows, which left the chip idle for a chunk of few rows (us a launch; rows x keys,
+// heads): 504 x 20,984, 32: 112 -> 54 (64 heads 158 -> 85); 1024 x 8192, 64: 125 -> 63; 904 x 5003, 64:
+// 79 -> 39; 64 x 60,064, 64: 227 -> 38; 16 x 30,016, 64: 224 -> 8.6; 2048 x 32,048, 32: 266 -> 242; a
+// 4096-row slab over 69,632 keys is the same for every L (1812-1822).  Over a sweep of L at each
+// shape the rule's time is within 7% of the best.
+int64_t slice_pages_for(int64_t n_groups, int64_t width_pages, int64_t n_cu, int64_t max_pages) {
+  int64_t best = 1, best_cost = INT64_MAX;
+  for (int64_t L = 1; L <= std::min(max_pages, width_pages); ++L) {
+    const int64_t rounds = (n_groups * ((width_pages + L - 1) / L) + n_cu - 1) / n_cu;
+    const int64_t cost = rounds * (L + 1) * (rounds == 1 ? 8 : 6) + 3 * L;  // in sixths of a page
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = L;
+    }
+  }
+  return best;
+}
+
 // Enqueues the kernel for a.batch rows in groups of R (a.group rows share a block-table row;
 // a.width caps the lengths).  a's pointers, strides and sizes are set and checked by the caller.
 int enqueue(DecodeArgs a, int heads, int R, int target_ctas, bool hist, const int32_t* hist_lens, int32_t* hist_ws,
@@ -679,15 +658,16 @@ int enqueue(DecodeArgs a, int heads, int R, int target_ctas, bool hist, const in
   a.slice_pages = 0;
   const int64_t width_pages = (a.width + kPage - 1) / kPage;
   // (the maskless eight-row instantiation is the one that carries the slice-major assignment)
-  if (slice_major && R == 8 && a.mask == nullptr && width_pages <= static_cast<int64_t>(kMaxSlices) * max_cta_pages) {
-    // slices as long as the block-table stage allows (the balanced grid's slice length at these
-    // shapes), a CTA per (slice, group) pair the widest group could need
-    const int64_t n_sl = (width_pages + max_cta_pages - 1) / max_cta_pages;
+  if (slice_major && R == 8 && a.mask == nullptr) {
+    int n_cu = 0;
+    const int st = dsa_device_cu_count(&n_cu);
+    if (st != DSA_OK) return st;
+    a.slice_pages = static_cast<int>(slice_pages_for(n_groups, width_pages, n_cu, max_cta_pages));
+    const int64_t n_sl = (width_pages + a.slice_pages - 1) / a.slice_pages;
     const int64_t grid = n_groups * n_sl;
     DSA_REQUIRE(grid <= 0x7FFFFFFF, "%s: grid too large", who);
     a.R = R;
     a.n_groups = static_cast<int>(n_groups);
-    a.slice_pages = static_cast<int>((width_pages + n_sl - 1) / n_sl);
     a.nt_logits = a.batch * static_cast<int64_t>(a.width) * 4 > (16ll << 20) ? 1 : 0;
     a.target = 0;
     a.hist_lens = nullptr;
