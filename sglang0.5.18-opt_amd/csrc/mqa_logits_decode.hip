@@ -326,12 +326,16 @@ __global__ __launch_bounds__((Shape<R, kHist>::kThreads)) __attribute__((amdgpu_
   const int r = wave / S;
   const int s = wave % S;
   const int row0 = grp * R;
-  const int row = row0 + r;
+  // The last group of a prefill may be short of R rows: a wave past the last row has length 0 (it takes
+  // its share of the page DMAs and the barriers and scores nothing), its reads go to the last row.
+  const int last = static_cast<int>(a.batch) - 1;
+  const bool in_batch = kMask || row0 + r <= last;  // wave-uniform
+  const int row = in_batch ? row0 + r : last;
   const int group_row = (row0 / a.group) * a.group;
   int max_len = 0;
 #pragma unroll
-  for (int q = 0; q < R; ++q) max_len = max(max_len, clamp_len(a.ctx[row0 + q], a.width));
-  const int len = clamp_len(a.ctx[row], a.width);
+  for (int q = 0; q < R; ++q) max_len = max(max_len, clamp_len(a.ctx[kMask ? row0 + q : min(row0 + q, last)], a.width));
+  const int len = in_batch ? clamp_len(a.ctx[row], a.width) : 0;
   int hlim = 0;
   if constexpr (kHist) {
     int h = a.hist_lens[row];
@@ -349,6 +353,8 @@ __global__ __launch_bounds__((Shape<R, kHist>::kThreads)) __attribute__((amdgpu_
     p_end = static_cast<int>(static_cast<int64_t>(pages) * (jc + 1) / nj);
   }
   const int n_local = p_end - p_begin;  // <= Sh::kMaxPages by the host's choice of target
+  // the pages this wave scores: without a mask to write, those that hold tokens of its row
+  const int n_mine = kMask ? n_local : min(n_local, (len + kPage - 1) / kPage - p_begin);
   const int32_t* btr = a.bt + static_cast<int64_t>(group_row) * a.bt_stride + p_begin;
 
   // The block-table entries of the stream's first two pages, read together and waited for
@@ -470,7 +476,7 @@ __global__ __launch_bounds__((Shape<R, kHist>::kThreads)) __attribute__((amdgpu_
       const int pg = __builtin_amdgcn_readfirstlane(s_bt[i + (NS - 1) * S]);
       dma_page<R>(a.kv + static_cast<int64_t>(pg) * a.page_stride, nxt, r, lane);
     }
-    if (i >= n_local) return;  // stream-uniform (the stream still takes part in the barriers)
+    if (i >= n_mine) return;  // wave-uniform (the wave still takes part in the barriers)
     const float scale = reinterpret_cast<const float*>(cur + kPageFp8Bytes)[lane];
     float part[4];  // this lane's heads' share of tokens st * 16 + lane % 16
     // One-row CTAs read the page's four K fragments from LDS before the first MFMA, instead of
@@ -650,34 +656,12 @@ int64_t slice_pages_for(int64_t n_groups, int64_t width_pages, int64_t n_cu, int
 // Enqueues the kernel for a.batch rows in groups of R (a.group rows share a block-table row;
 // a.width caps the lengths).  a's pointers, strides and sizes are set and checked by the caller.
 int enqueue(DecodeArgs a, int heads, int R, int target_ctas, bool hist, const int32_t* hist_lens, int32_t* hist_ws,
-            hipStream_t stream, const char* who, bool slice_major = false) {
+            hipStream_t stream, const char* who) {
   const int64_t n_groups = a.batch / R;
   DSA_REQUIRE(n_groups <= 0x3FFFFFFF, "%s: too many rows", who);
   int ctas_per_cu = 1, max_cta_pages = 1;
   shape_host(R, hist, ctas_per_cu, max_cta_pages);
   a.slice_pages = 0;
-  const int64_t width_pages = (a.width + kPage - 1) / kPage;
-  // (the maskless eight-row instantiation is the one that carries the slice-major assignment)
-  if (slice_major && R == 8 && a.mask == nullptr) {
-    int n_cu = 0;
-    const int st = dsa_device_cu_count(&n_cu);
-    if (st != DSA_OK) return st;
-    a.slice_pages = static_cast<int>(slice_pages_for(n_groups, width_pages, n_cu, max_cta_pages));
-    const int64_t n_sl = (width_pages + a.slice_pages - 1) / a.slice_pages;
-    const int64_t grid = n_groups * n_sl;
-    DSA_REQUIRE(grid <= 0x7FFFFFFF, "%s: grid too large", who);
-    a.R = R;
-    a.n_groups = static_cast<int>(n_groups);
-    a.nt_logits = a.batch * static_cast<int64_t>(a.width) * 4 > (16ll << 20) ? 1 : 0;
-    a.target = 0;
-    a.hist_lens = nullptr;
-    a.hist_ws = nullptr;
-    a.zero_ws = nullptr;
-    const uint32_t g = static_cast<uint32_t>(grid);
-    if (heads == 64) launch_r<64, false>(a, R, g, stream);
-    else launch_r<32, false>(a, R, g, stream);
-    return check_launch(who);
-  }
   if (target_ctas <= 0) {
     // All CTAs resident at once: the per-group rounding adds up to one CTA per group, so aim
     // below the resident count by the group count.
@@ -723,6 +707,28 @@ int enqueue(DecodeArgs a, int heads, int R, int target_ctas, bool hist, const in
     if (hist) launch_r<32, true>(a, R, g, stream);
     else launch_r<32, false>(a, R, g, stream);
   }
+  return check_launch(who);
+}
+
+// The same for a.batch rows of one request in groups of 8 (the last one may be short), no mask: the
+// (slice, group) pairs of slice_pages_for.
+int enqueue_slices(DecodeArgs a, int heads, hipStream_t stream, const char* who) {
+  constexpr int R = 8;
+  const int64_t n_groups = (a.batch + R - 1) / R;
+  int ctas_per_cu = 1, max_cta_pages = 1, n_cu = 0;
+  shape_host(R, false, ctas_per_cu, max_cta_pages);
+  const int st = dsa_device_cu_count(&n_cu);
+  if (st != DSA_OK) return st;
+  const int64_t width_pages = (a.width + kPage - 1) / kPage;
+  a.slice_pages = static_cast<int>(slice_pages_for(n_groups, width_pages, n_cu, max_cta_pages));
+  const int64_t grid = n_groups * ((width_pages + a.slice_pages - 1) / a.slice_pages);
+  DSA_REQUIRE(grid <= 0x7FFFFFFF, "%s: grid too large", who);
+  a.R = R;
+  a.n_groups = static_cast<int>(n_groups);
+  a.nt_logits = a.batch * static_cast<int64_t>(a.width) * 4 > (16ll << 20) ? 1 : 0;
+  const uint32_t g = static_cast<uint32_t>(grid);
+  if (heads == 64) launch_r<64, false>(a, R, g, stream);
+  else launch_r<32, false>(a, R, g, stream);
   return check_launch(who);
 }
 
@@ -785,8 +791,11 @@ extern "C" int dsa_mqa_logits_decode(const uint8_t* q8, const float* w, int head
 
 // Prefill: the rows of one request are one group sharing the request's block table, scored by
 // the same kernel in CTAs of 8 rows (8 waves on one LDS page stream: each K page read from HBM
-// once per 8 query rows); a row count that is not a multiple of 8 ends in groups of 4 and of
-// 1-3 rows, each its own launch.  No mask is written.
+// once per 8 query rows), the last group short when the count is not a multiple of 8: launches of their
+// own for a remainder's 4, 2 and 1 rows read the whole of K again, one after the other (us, launches of
+// their own -> one short group, 64 heads: 7 x 3007 12.1 -> 5.3; 39 x 1039 16.6 -> 5.3; 15 x 100,015 37.1
+// -> 19.2; 5 x 30,005 10.3 -> 7.6; 509 x 20,989, 32 heads 62 -> 54).  Up to 4 rows take the decode grid
+// in groups of 4, 2 and 1 (4 x 30,004: 6.0).  No mask is written.
 extern "C" int dsa_mqa_logits_prefill(const uint8_t* q8, const float* w, int heads, int64_t rows,
                                       const uint8_t* kv_cache, int64_t page_stride_bytes, const int32_t* block_table,
                                       int64_t bt_pages, const int32_t* lens, float* logits, int64_t logits_stride,
@@ -803,7 +812,8 @@ extern "C" int dsa_mqa_logits_prefill(const uint8_t* q8, const float* w, int hea
               "dsa_mqa_logits_prefill: kv_cache pages (stride >= 8448, %% 16) and q8 must be 16-B aligned");
   int64_t done = 0;
   for (const int R : {8, 4, 2, 1}) {
-    const int64_t n = (rows - done) / R * R;
+    const int64_t left = rows - done;
+    const int64_t n = R == 8 ? (left > 4 ? left : 0) : left / R * R;
     if (n == 0) continue;
     DecodeArgs a{};
     a.q8 = q8 + done * heads * kHeadDim;
@@ -821,7 +831,8 @@ extern "C" int dsa_mqa_logits_prefill(const uint8_t* q8, const float* w, int hea
     a.mask_stride = 0;
     a.group = static_cast<int>(n);
     a.batch = n;
-    const int st = enqueue(a, heads, R, 0, false, nullptr, nullptr, stream, "dsa_mqa_logits_prefill", true);
+    const int st = R == 8 ? enqueue_slices(a, heads, stream, "dsa_mqa_logits_prefill")
+                          : enqueue(a, heads, R, 0, false, nullptr, nullptr, stream, "dsa_mqa_logits_prefill");
     if (st != DSA_OK) return st;
     done += n;
   }
