@@ -252,6 +252,12 @@ namespace dsa {
 int fail(int code, const char* fmt, ...);
 int ok();
 int check_launch(const char* what);
+
+// dsa_topk_transform of dense scores whose rows may be read up to `cols` >= width floats (the pad of a
+// row, its values unused).
+int topk_padded(const float* score, int64_t score_stride, int64_t width, int64_t cols, const int32_t* lengths,
+                int64_t rows, const int32_t* page_table, int64_t pt_stride, int64_t pt_cols, int max_splits, int n_cu,
+                void* workspace, size_t workspace_bytes, int32_t* out, hipStream_t stream, const char* who);
 }  // namespace dsa
 
 #define DSA_REQUIRE(cond, ...)                                      \

@@ -1833,8 +1833,9 @@ WsLayout ws_layout(int64_t rows, int cap) {
   return l;
 }
 
-// pt_cols: entries per page-table row; pt_shift 6: the entries are 64-token pages (PtRow).
-int topk_common(const float* score, int64_t score_stride, int64_t width, const int16_t* mask, int64_t mask_stride,
+// cols: floats of a score row that may be read (>= width); pt_cols: entries per page-table row;
+// pt_shift 6: the entries are 64-token pages (PtRow).
+int topk_common(const float* score, int64_t score_stride, int64_t width, int64_t cols, const int16_t* mask, int64_t mask_stride,
                 const int32_t* lengths, int64_t rows, const int32_t* page_table, int64_t pt_stride, int64_t pt_cols,
                 int pt_shift, const int32_t* cu_seqlens_q, int64_t n_req, int max_splits, int n_cu,
                 int32_t* pre_hist, bool pass1_done, void* workspace, size_t workspace_bytes, int32_t* out,
@@ -1852,7 +1853,8 @@ int topk_common(const float* score, int64_t score_stride, int64_t width, const i
   DSA_REQUIRE(pt_cols >= 0 && pt_cols <= 0x7FFFFFFF && (pt_stride >= pt_cols || pt_stride == 0),
               "%s: page-table row stride < its entries per row (and not 0)", who);
   DSA_REQUIRE(pt_shift == 0 || pt_shift == 6, "%s: page-table entries cover 1 or 64 tokens", who);
-  const bool vec = width % 4 == 0 && score_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(score) & 15u) == 0;
+  // 16-B loads: a row's last quad, the one its length may end in, lies inside the row's cols floats
+  const bool vec = cols % 4 == 0 && score_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(score) & 15u) == 0;
 
   TopkArgs a;
   a.score = score;
@@ -1944,6 +1946,14 @@ int topk_common(const float* score, int64_t score_stride, int64_t width, const i
 }
 
 }  // namespace
+
+int topk_padded(const float* score, int64_t score_stride, int64_t width, int64_t cols, const int32_t* lengths,
+                int64_t rows, const int32_t* page_table, int64_t pt_stride, int64_t pt_cols, int max_splits, int n_cu,
+                void* workspace, size_t workspace_bytes, int32_t* out, hipStream_t stream, const char* who) {
+  return topk_common(score, score_stride, width, cols, nullptr, 0, lengths, rows, page_table, pt_stride, pt_cols, 0,
+                     nullptr, rows, max_splits, n_cu, nullptr, false, workspace, workspace_bytes, out, stream, who);
+}
+
 }  // namespace dsa
 
 using namespace dsa;
@@ -1963,7 +1973,7 @@ extern "C" int dsa_topk_transform(const float* score, int64_t score_stride, int6
                                   const int32_t* page_table, int64_t pt_stride, int64_t pt_cols,
                                   const int32_t* cu_seqlens_q, int64_t n_req, int max_splits, int n_cu,
                                   void* workspace, size_t workspace_bytes, int32_t* out, hipStream_t stream) {
-  return topk_common(score, score_stride, width, mask, mask_stride, lengths, rows, page_table, pt_stride, pt_cols, 0,
+  return topk_common(score, score_stride, width, width, mask, mask_stride, lengths, rows, page_table, pt_stride, pt_cols, 0,
                      cu_seqlens_q, n_req, max_splits, n_cu, nullptr, false, workspace, workspace_bytes, out, stream,
                      "dsa_topk_transform");
 }
@@ -1975,7 +1985,7 @@ extern "C" int dsa_topk_transform_pre(const float* score, int64_t score_stride, 
                                       int32_t* hist_ws, int pass1_done, void* workspace, size_t workspace_bytes,
                                       int32_t* out, hipStream_t stream) {
   DSA_REQUIRE(hist_ws != nullptr, "dsa_topk_transform_pre: hist_ws is null");
-  return topk_common(score, score_stride, width, mask, mask_stride, lengths, rows, page_table, pt_stride, pt_cols, 0,
+  return topk_common(score, score_stride, width, width, mask, mask_stride, lengths, rows, page_table, pt_stride, pt_cols, 0,
                      cu_seqlens_q, n_req, max_splits, n_cu, hist_ws, pass1_done != 0, workspace, workspace_bytes, out,
                      stream, "dsa_topk_transform_pre");
 }
@@ -1986,7 +1996,7 @@ extern "C" int dsa_topk_transform_blocks(const float* score, int64_t score_strid
                                          const int32_t* cu_seqlens_q, int64_t n_req, int max_splits, int n_cu,
                                          int32_t* hist_ws, int pass1_done, void* workspace, size_t workspace_bytes,
                                          int32_t* out, hipStream_t stream) {
-  return topk_common(score, score_stride, width, mask, mask_stride, lengths, rows, block_table, bt_stride, bt_pages,
+  return topk_common(score, score_stride, width, width, mask, mask_stride, lengths, rows, block_table, bt_stride, bt_pages,
                      6, cu_seqlens_q, n_req, max_splits, n_cu, hist_ws, hist_ws != nullptr && pass1_done != 0,
                      workspace, workspace_bytes, out, stream, "dsa_topk_transform_blocks");
 }
@@ -2052,6 +2062,6 @@ extern "C" int dsa_topk_transform_noalloc(const float* score, int64_t score_stri
     const int st = scratch_address(&ws, who);
     if (st != DSA_OK) return st;
   }
-  return topk_common(score, score_stride, width, mask, mask_stride, lengths, rows, page_table, pt_stride, pt_cols, 0,
+  return topk_common(score, score_stride, width, width, mask, mask_stride, lengths, rows, page_table, pt_stride, pt_cols, 0,
                      cu_seqlens_q, n_req, max_splits, n_cu, nullptr, false, ws, need, out, stream, who);
 }
