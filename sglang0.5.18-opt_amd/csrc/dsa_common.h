@@ -253,6 +253,12 @@ int fail(int code, const char* fmt, ...);
 int ok();
 int check_launch(const char* what);
 
+// dsa_mqa_logits_prefill that may leave out the logits of rows of at most min_len keys (no caller reads
+// them: such a row selects all of its keys).
+int mqa_logits_prefill_over(const uint8_t* q8, const float* w, int heads, int64_t rows, const uint8_t* kv_cache,
+                            int64_t page_stride_bytes, const int32_t* block_table, int64_t bt_pages,
+                            const int32_t* lens, float* logits, int64_t logits_stride, int64_t width, int min_len,
+                            hipStream_t stream);
 // dsa_topk_transform of dense scores whose rows may be read up to `cols` >= width floats (the pad of a
 // row, its values unused).
 int topk_padded(const float* score, int64_t score_stride, int64_t width, int64_t cols, const int32_t* lengths,

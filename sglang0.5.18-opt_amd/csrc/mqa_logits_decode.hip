@@ -120,10 +120,18 @@ struct DecodeArgs {
   int32_t* zero_ws;   // non-null: the paired top-k's workspace, whose counters are zeroed here
   int64_t batch;
   int nt_logits;      // logits stored nontemporally (a logits block larger than the L2s hold)
+  int min_len;        // eight-row prefill: rows of at most this many tokens are not scored
   int slice_pages;    // > 0: slice-major assignment with slices of this many pages
 };
 
 __device__ __forceinline__ int clamp_len(int l, int width) { return l < 0 ? 0 : (l > width ? width : l); }
+
+// The tokens of a row that are scored (kMask: every row; else those of rows past min_len).
+template <bool kMask>
+__device__ __forceinline__ int scored_len(const DecodeArgs& a, int row) {
+  const int l = clamp_len(a.ctx[row], a.width);
+  return kMask || l > a.min_len ? l : 0;
+}
 
 // Pages of row group g: ceil(max over its R rows of len / 64).
 __device__ __forceinline__ int group_pages(const DecodeArgs& a, int g) {
@@ -334,8 +342,8 @@ __global__ __launch_bounds__((Shape<R, kHist>::kThreads)) __attribute__((amdgpu_
   const int group_row = (row0 / a.group) * a.group;
   int max_len = 0;
 #pragma unroll
-  for (int q = 0; q < R; ++q) max_len = max(max_len, clamp_len(a.ctx[kMask ? row0 + q : min(row0 + q, last)], a.width));
-  const int len = in_batch ? clamp_len(a.ctx[row], a.width) : 0;
+  for (int q = 0; q < R; ++q) max_len = max(max_len, scored_len<kMask>(a, kMask ? row0 + q : min(row0 + q, last)));
+  const int len = in_batch ? scored_len<kMask>(a, row) : 0;
   int hlim = 0;
   if constexpr (kHist) {
     int h = a.hist_lens[row];
@@ -796,10 +804,10 @@ extern "C" int dsa_mqa_logits_decode(const uint8_t* q8, const float* w, int head
 // their own -> one short group, 64 heads: 7 x 3007 12.1 -> 5.3; 39 x 1039 16.6 -> 5.3; 15 x 100,015 37.1
 // -> 19.2; 5 x 30,005 10.3 -> 7.6; 509 x 20,989, 32 heads 62 -> 54).  Up to 4 rows take the decode grid
 // in groups of 4, 2 and 1 (4 x 30,004: 6.0).  No mask is written.
-extern "C" int dsa_mqa_logits_prefill(const uint8_t* q8, const float* w, int heads, int64_t rows,
-                                      const uint8_t* kv_cache, int64_t page_stride_bytes, const int32_t* block_table,
-                                      int64_t bt_pages, const int32_t* lens, float* logits, int64_t logits_stride,
-                                      int64_t width, hipStream_t stream) {
+int dsa::mqa_logits_prefill_over(const uint8_t* q8, const float* w, int heads, int64_t rows, const uint8_t* kv_cache,
+                                 int64_t page_stride_bytes, const int32_t* block_table, int64_t bt_pages,
+                                 const int32_t* lens, float* logits, int64_t logits_stride, int64_t width,
+                                 int min_len, hipStream_t stream) {
   DSA_REQUIRE(heads == 32 || heads == 64, "dsa_mqa_logits_prefill: heads must be 32 or 64 (got %d)", heads);
   DSA_REQUIRE(rows >= 0 && rows <= 0x7FFFFFFF, "dsa_mqa_logits_prefill: rows out of range");
   if (rows == 0) return ok();
@@ -810,6 +818,7 @@ extern "C" int dsa_mqa_logits_prefill(const uint8_t* q8, const float* w, int hea
   DSA_REQUIRE(page_stride_bytes >= kPageBytes && page_stride_bytes % 16 == 0 &&
                   (reinterpret_cast<uintptr_t>(kv_cache) & 15u) == 0 && (reinterpret_cast<uintptr_t>(q8) & 15u) == 0,
               "dsa_mqa_logits_prefill: kv_cache pages (stride >= 8448, %% 16) and q8 must be 16-B aligned");
+  if (width <= min_len) return ok();  // no row is longer
   int64_t done = 0;
   for (const int R : {8, 4, 2, 1}) {
     const int64_t left = rows - done;
@@ -831,10 +840,19 @@ extern "C" int dsa_mqa_logits_prefill(const uint8_t* q8, const float* w, int hea
     a.mask_stride = 0;
     a.group = static_cast<int>(n);
     a.batch = n;
+    a.min_len = min_len;
     const int st = R == 8 ? enqueue_slices(a, heads, stream, "dsa_mqa_logits_prefill")
                           : enqueue(a, heads, R, 0, false, nullptr, nullptr, stream, "dsa_mqa_logits_prefill");
     if (st != DSA_OK) return st;
     done += n;
   }
   return ok();
+}
+
+extern "C" int dsa_mqa_logits_prefill(const uint8_t* q8, const float* w, int heads, int64_t rows,
+                                      const uint8_t* kv_cache, int64_t page_stride_bytes, const int32_t* block_table,
+                                      int64_t bt_pages, const int32_t* lens, float* logits, int64_t logits_stride,
+                                      int64_t width, hipStream_t stream) {
+  return mqa_logits_prefill_over(q8, w, heads, rows, kv_cache, page_stride_bytes, block_table, bt_pages, lens, logits,
+                                 logits_stride, width, 0, stream);
 }

@@ -88,9 +88,10 @@ extern "C" int dsa_prefill_indexer(const uint8_t* q8, const float* w, int heads,
   const size_t topk_bytes = workspace_bytes - (topk_ws - static_cast<char*>(workspace));
   for (int64_t r0 = 0; r0 < rows; r0 += s) {
     const int64_t n = rows - r0 < s ? rows - r0 : s;
-    int st = dsa_mqa_logits_prefill(q8 + r0 * heads * kHeadDim, w + r0 * heads, heads, n, kv_cache,
-                                    page_stride_bytes, block_table, bt_pages, lens + r0, logits, stride, width,
-                                    stream);
+    // a row of at most 2048 keys selects all of them, so its logits are left out (64 heads, whole call:
+    // a prompt of 2048 tokens 57.6 -> 27.0 us, of 5003 262 -> 248, 1000 rows over 1500 keys 64.7 -> 56.9)
+    int st = mqa_logits_prefill_over(q8 + r0 * heads * kHeadDim, w + r0 * heads, heads, n, kv_cache, page_stride_bytes,
+                                     block_table, bt_pages, lens + r0, logits, stride, width, kTopK, stream);
     if (st != DSA_OK) return st;
     // every row of the request reads the same page-table row (row stride 0)
     st = topk_padded(logits, stride, width, stride, lens + r0, n, page_table, 0, pt_cols, max_splits, n_cu, topk_ws,
