@@ -227,7 +227,9 @@ int dsa_topk_transform_blocks(const float* score, int64_t score_stride, int64_t 
  * q8 / w / kv_cache / block_table / lens as in dsa_mqa_logits_prefill; out int32 [rows, 2048].
  * dsa_prefill_slab_rows gives the slab size a byte budget of logits allows (a multiple of 8
  * rows when at least 8 fit, capped at max_slab_rows > 0 and at rows);
- * dsa_prefill_indexer_workspace_bytes the workspace (256-B aligned) the call needs. */
+ * dsa_prefill_indexer_workspace_bytes the workspace (256-B aligned) for rows padded to 128 B; one
+ * without room for the pad (the logits slab of `width` floats a row, up to 256 B, then the top-k's
+ * workspace) is taken too and holds unpadded rows. */
 int64_t dsa_prefill_slab_rows(int64_t rows, int64_t width, int64_t max_slab_rows, int64_t memory_budget_bytes);
 size_t dsa_prefill_indexer_workspace_bytes(int64_t rows, int64_t width, int64_t slab_rows, int max_splits,
                                            int n_cu);
@@ -236,6 +238,12 @@ int dsa_prefill_indexer(const uint8_t* q8, const float* w, int heads, int64_t ro
                         const int32_t* lens, int64_t width, const int32_t* page_table, int64_t pt_cols,
                         int64_t slab_rows, int max_splits, int n_cu, void* workspace, size_t workspace_bytes,
                         int32_t* out, hipStream_t stream);
+/* dsa_prefill_indexer with the block table's own slots as the page table: token t maps to
+ * block_table[t / 64] * 64 + t % 64 (for callers without an expanded table). */
+int dsa_prefill_indexer_blocks(const uint8_t* q8, const float* w, int heads, int64_t rows, const uint8_t* kv_cache,
+                               int64_t page_stride_bytes, const int32_t* block_table, int64_t bt_pages,
+                               const int32_t* lens, int64_t width, int64_t slab_rows, int max_splits, int n_cu,
+                               void* workspace, size_t workspace_bytes, int32_t* out, hipStream_t stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Diagnostic, no counterpart in the reference: the fp8 MFMA throughput the chip reaches, the

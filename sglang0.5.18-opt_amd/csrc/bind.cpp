@@ -331,11 +331,12 @@ torch::Tensor mqa_logits_prefill(const torch::Tensor& q, const torch::Tensor& we
 
 // Prefill indexer of one request (dsa_prefill_indexer): logits in slabs of at most
 // max_slab_rows rows and memory_budget_bytes of f32 logits, each slab's top-2048 behind it.
-// page_table_1: int32 [>= width] token -> slot of the request (the remap of the output).
+// page_table_1: int32 [>= width] token -> slot of the request (the remap of the output); None: the block
+// table's slots.
 torch::Tensor prefill_indexer(const torch::Tensor& q, const torch::Tensor& weights, const torch::Tensor& kv_cache,
                               const torch::Tensor& block_table, const torch::Tensor& lens, int64_t width,
-                              const torch::Tensor& page_table_1, int64_t memory_budget_bytes, int64_t max_slab_rows,
-                              int64_t max_splits, const c10::optional<torch::Tensor>& out) {
+                              const c10::optional<torch::Tensor>& page_table_1, int64_t memory_budget_bytes,
+                              int64_t max_slab_rows, int64_t max_splits, const c10::optional<torch::Tensor>& out) {
   TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::kFloat8_e4m3fn && q.dim() == 3 &&
                   (q.size(1) == 32 || q.size(1) == 64) && q.size(2) == kHeadDim && q.is_contiguous(),
               "q must be contiguous fp8 e4m3fn [rows, H, 128] with H in {32, 64}");
@@ -349,7 +350,8 @@ torch::Tensor prefill_indexer(const torch::Tensor& q, const torch::Tensor& weigh
               "block_table must be contiguous int32 [pages]");
   TORCH_CHECK(lens.scalar_type() == at::kInt && lens.dim() == 1 && lens.size(0) == rows && lens.is_contiguous(),
               "lens must be contiguous int32 [rows]");
-  TORCH_CHECK(page_table_1.scalar_type() == at::kInt && page_table_1.dim() == 1 && page_table_1.is_contiguous(),
+  TORCH_CHECK(!page_table_1.has_value() || (page_table_1->scalar_type() == at::kInt && page_table_1->dim() == 1 &&
+                                            page_table_1->is_contiguous()),
               "page_table_1 must be contiguous int32 [tokens]");
   TORCH_CHECK(width > 0 && width <= block_table.size(0) * kPage, "width must be within the block table capacity");
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
@@ -368,11 +370,19 @@ torch::Tensor prefill_indexer(const torch::Tensor& q, const torch::Tensor& weigh
   const int64_t slab = dsa_prefill_slab_rows(rows, width, max_slab_rows, memory_budget_bytes);
   const size_t ws_bytes = dsa_prefill_indexer_workspace_bytes(rows, width, slab, splits, cus);
   auto ws = torch::empty({static_cast<int64_t>(ws_bytes)}, q.options().dtype(at::kByte));
-  check_status(dsa_prefill_indexer(reinterpret_cast<const uint8_t*>(q.data_ptr()), weights.data_ptr<float>(),
-                                   static_cast<int>(H), rows, kv_cache.data_ptr<uint8_t>(), kv_cache.stride(0),
-                                   block_table.data_ptr<int>(), block_table.size(0), lens.data_ptr<int>(), width,
-                                   page_table_1.data_ptr<int>(), page_table_1.size(0), slab, splits, cus,
-                                   ws.data_ptr(), ws_bytes, dst.data_ptr<int>(), cur_stream()));
+  const uint8_t* q8 = reinterpret_cast<const uint8_t*>(q.data_ptr());
+  if (page_table_1.has_value()) {
+    check_status(dsa_prefill_indexer(q8, weights.data_ptr<float>(), static_cast<int>(H), rows,
+                                     kv_cache.data_ptr<uint8_t>(), kv_cache.stride(0), block_table.data_ptr<int>(),
+                                     block_table.size(0), lens.data_ptr<int>(), width, page_table_1->data_ptr<int>(),
+                                     page_table_1->size(0), slab, splits, cus, ws.data_ptr(), ws_bytes,
+                                     dst.data_ptr<int>(), cur_stream()));
+  } else {
+    check_status(dsa_prefill_indexer_blocks(
+        q8, weights.data_ptr<float>(), static_cast<int>(H), rows, kv_cache.data_ptr<uint8_t>(), kv_cache.stride(0),
+        block_table.data_ptr<int>(), block_table.size(0), lens.data_ptr<int>(), width, slab, splits, cus,
+        ws.data_ptr(), ws_bytes, dst.data_ptr<int>(), cur_stream()));
+  }
   return dst;
 }
 

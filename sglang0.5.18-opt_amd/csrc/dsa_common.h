@@ -260,10 +260,11 @@ int mqa_logits_prefill_over(const uint8_t* q8, const float* w, int heads, int64_
                             const int32_t* lens, float* logits, int64_t logits_stride, int64_t width, int min_len,
                             hipStream_t stream);
 // dsa_topk_transform of dense scores whose rows may be read up to `cols` >= width floats (the pad of a
-// row, its values unused).
+// row, its values unused); pt_shift 6: page_table is a block table of 64-token pages.
 int topk_padded(const float* score, int64_t score_stride, int64_t width, int64_t cols, const int32_t* lengths,
-                int64_t rows, const int32_t* page_table, int64_t pt_stride, int64_t pt_cols, int max_splits, int n_cu,
-                void* workspace, size_t workspace_bytes, int32_t* out, hipStream_t stream, const char* who);
+                int64_t rows, const int32_t* page_table, int64_t pt_stride, int64_t pt_cols, int pt_shift,
+                int max_splits, int n_cu, void* workspace, size_t workspace_bytes, int32_t* out, hipStream_t stream,
+                const char* who);
 }  // namespace dsa
 
 #define DSA_REQUIRE(cond, ...)                                      \

@@ -64,11 +64,12 @@ extern "C" size_t dsa_prefill_indexer_workspace_bytes(int64_t rows, int64_t widt
   return workspace_bytes_of(rows, width, slab_stride(width), slab_rows < rows ? slab_rows : rows, max_splits, n_cu);
 }
 
-extern "C" int dsa_prefill_indexer(const uint8_t* q8, const float* w, int heads, int64_t rows,
-                                   const uint8_t* kv_cache, int64_t page_stride_bytes, const int32_t* block_table,
-                                   int64_t bt_pages, const int32_t* lens, int64_t width, const int32_t* page_table,
-                                   int64_t pt_cols, int64_t slab_rows, int max_splits, int n_cu, void* workspace,
-                                   size_t workspace_bytes, int32_t* out, hipStream_t stream) {
+// The slab loop; pt_shift 6: page_table is the block table itself (pt_cols pages).
+static int prefill_indexer(const uint8_t* q8, const float* w, int heads, int64_t rows, const uint8_t* kv_cache,
+                           int64_t page_stride_bytes, const int32_t* block_table, int64_t bt_pages,
+                           const int32_t* lens, int64_t width, const int32_t* page_table, int64_t pt_cols, int pt_shift,
+                           int64_t slab_rows, int max_splits, int n_cu, void* workspace, size_t workspace_bytes,
+                           int32_t* out, hipStream_t stream) {
   DSA_REQUIRE(rows >= 0 && width > 0 && width <= 0x7FFFFFFF, "dsa_prefill_indexer: rows / width out of range");
   if (rows == 0) return ok();
   DSA_REQUIRE(slab_rows >= 1, "dsa_prefill_indexer: slab_rows must be >= 1");
@@ -94,9 +95,28 @@ extern "C" int dsa_prefill_indexer(const uint8_t* q8, const float* w, int heads,
                                      block_table, bt_pages, lens + r0, logits, stride, width, kTopK, stream);
     if (st != DSA_OK) return st;
     // every row of the request reads the same page-table row (row stride 0)
-    st = topk_padded(logits, stride, width, stride, lens + r0, n, page_table, 0, pt_cols, max_splits, n_cu, topk_ws,
-                     topk_bytes, out + r0 * kTopK, stream, "dsa_prefill_indexer");
+    st = topk_padded(logits, stride, width, stride, lens + r0, n, page_table, 0, pt_cols, pt_shift, max_splits, n_cu,
+                     topk_ws, topk_bytes, out + r0 * kTopK, stream, "dsa_prefill_indexer");
     if (st != DSA_OK) return st;
   }
   return ok();
+}
+
+extern "C" int dsa_prefill_indexer(const uint8_t* q8, const float* w, int heads, int64_t rows,
+                                   const uint8_t* kv_cache, int64_t page_stride_bytes, const int32_t* block_table,
+                                   int64_t bt_pages, const int32_t* lens, int64_t width, const int32_t* page_table,
+                                   int64_t pt_cols, int64_t slab_rows, int max_splits, int n_cu, void* workspace,
+                                   size_t workspace_bytes, int32_t* out, hipStream_t stream) {
+  return prefill_indexer(q8, w, heads, rows, kv_cache, page_stride_bytes, block_table, bt_pages, lens, width,
+                         page_table, pt_cols, 0, slab_rows, max_splits, n_cu, workspace, workspace_bytes, out, stream);
+}
+
+extern "C" int dsa_prefill_indexer_blocks(const uint8_t* q8, const float* w, int heads, int64_t rows,
+                                          const uint8_t* kv_cache, int64_t page_stride_bytes,
+                                          const int32_t* block_table, int64_t bt_pages, const int32_t* lens,
+                                          int64_t width, int64_t slab_rows, int max_splits, int n_cu, void* workspace,
+                                          size_t workspace_bytes, int32_t* out, hipStream_t stream) {
+  return prefill_indexer(q8, w, heads, rows, kv_cache, page_stride_bytes, block_table, bt_pages, lens, width,
+                         block_table, bt_pages, 6, slab_rows, max_splits, n_cu, workspace, workspace_bytes, out,
+                         stream);
 }

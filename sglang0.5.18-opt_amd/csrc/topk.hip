@@ -1948,10 +1948,11 @@ int topk_common(const float* score, int64_t score_stride, int64_t width, int64_t
 }  // namespace
 
 int topk_padded(const float* score, int64_t score_stride, int64_t width, int64_t cols, const int32_t* lengths,
-                int64_t rows, const int32_t* page_table, int64_t pt_stride, int64_t pt_cols, int max_splits, int n_cu,
-                void* workspace, size_t workspace_bytes, int32_t* out, hipStream_t stream, const char* who) {
-  return topk_common(score, score_stride, width, cols, nullptr, 0, lengths, rows, page_table, pt_stride, pt_cols, 0,
-                     nullptr, rows, max_splits, n_cu, nullptr, false, workspace, workspace_bytes, out, stream, who);
+                int64_t rows, const int32_t* page_table, int64_t pt_stride, int64_t pt_cols, int pt_shift,
+                int max_splits, int n_cu, void* workspace, size_t workspace_bytes, int32_t* out, hipStream_t stream,
+                const char* who) {
+  return topk_common(score, score_stride, width, cols, nullptr, 0, lengths, rows, page_table, pt_stride, pt_cols,
+                     pt_shift, nullptr, rows, max_splits, n_cu, nullptr, false, workspace, workspace_bytes, out, stream, who);
 }
 
 }  // namespace dsa
