@@ -99,7 +99,8 @@ int dsa_store_k_cache(const uint16_t* k_bf16, int64_t n_tokens, const int32_t* s
  * block_table [B, bt_pages] i32 with row stride bt_stride, width == bt_pages * 64 (mqa_hist.cu:346),
  * logits [B, width] f32 with row stride logits_stride; entries t >= len[r] are not written.
  * mask [B, width / 16] i16 with row stride mask_stride: every word is written.
- * heads in {32, 64}; B % group_size == 0; rows_per_cta divides group_size and is in {1,2,3,4,8}.
+ * heads in {32, 64}; B % group_size == 0; rows_per_cta divides group_size and is in {1,2,3,4,8}, or
+ * is <= 0: chosen from the sizes.
  * target_ctas: number of CTAs the K pages are spread over, each CTA streaming a slice of one
  * request (<= 0: as many as are resident at once); the grid is target_ctas + B / rows_per_cta.
  * hist_ws (nullable, int32 [B * (2 * 4096 + 2)], 16-B aligned): the pass-1 workspace of a

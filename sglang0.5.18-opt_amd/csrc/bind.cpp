@@ -93,7 +93,7 @@ std::vector<torch::Tensor> mqa_logits_hist(const torch::Tensor& q, const torch::
       reinterpret_cast<const uint8_t*>(q.data_ptr()), weights.data_ptr<float>(), static_cast<int>(H), B,
       static_cast<int>(group_size), kv_cache.data_ptr<uint8_t>(), kv_cache.stride(0), context_lens.data_ptr<int>(),
       block_table.data_ptr<int>(), block_table.stride(0), pages, logits.data_ptr<float>(), logits.stride(0),
-      mask.data_ptr<int16_t>(), mask_stride, static_cast<int>(R), target,
+      mask.data_ptr<int16_t>(), mask_stride, rows_per_cta > 0 ? static_cast<int>(R) : 0, target,
       hist ? hist_lens->data_ptr<int>() : nullptr, hist ? zws.data_ptr<int>() : nullptr, hist && fuse_pass1 ? 1 : 0,
       cur_stream()));
   return {logits, mask, zws};

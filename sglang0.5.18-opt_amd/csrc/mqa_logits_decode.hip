@@ -53,6 +53,7 @@ using u32x4 = __attribute__((ext_vector_type(4))) uint32_t;
 
 constexpr int kLdsBytes = 163840;  // LDS per CU
 constexpr int kMaxWavesCu = 16;    // waves per CU the register budget (<= 128 VGPRs) allows
+constexpr int kManyWavesCu = 24;   // the same for <= 80 VGPRs (32 heads, four rows a CTA and more)
 
 __device__ __forceinline__ f32x4 mfma_fp8(const i32x8& a, const i32x8& b, const f32x4& c) {
   // scale operands 0 select the unscaled v_mfma_f32_16x16x128_f8f6f4 (both operands fp8 e4m3)
@@ -238,15 +239,19 @@ __device__ __forceinline__ int3 assign_cta_wave(const DecodeArgs& a) {
 // MTP decode: one stream per CTA (eight CTAs per CU) without the histogram; with it, the 8 KB
 // per row of counters is amortised over two streams (R = 2) or four (R = 1).  One-row CTAs run
 // two streams (half the CTAs to dispatch for the same pages in flight: 32 x 16K decode 16.1 ->
-// 15.7 us, 1 x 4K 6.4 -> 6.3 us; two-row CTAs measured 0.5 us slower with two).
-template <int R, bool kHist>
+// 15.7 us, 1 x 4K 6.4 -> 6.3 us; two-row CTAs measured 0.5 us slower with two).  CTAs of four rows
+// and more hold few page streams a CU; with 32 heads they fit in 80 VGPRs, so six waves a SIMD (8
+// requests x 6 rows x 73,000 tokens, six-row CTAs: 28.5 us at 16 waves a CU, 24.7 at 24; a third or
+// fourth page slot per stream instead 26.9 and 31.3).
+template <int H, int R, bool kHist>
 struct Shape {
   static constexpr int S = kHist ? (R == 1 ? 4 : (R == 2 ? 2 : 1)) : (R == 1 ? 2 : 1);
   static constexpr int NS = 2;
   static constexpr int kMaxPages = S == 1 ? 255 : (S == 2 ? 511 : 1023);
   static constexpr int kLds = S * NS * kPageBytes + (kHist ? R * kBins * 2 : 0) + kMaxPages * 4 + 512;
   static constexpr int kByLds = kLdsBytes / kLds;
-  static constexpr int kByWaves = kMaxWavesCu / (R * S) > 0 ? kMaxWavesCu / (R * S) : 1;
+  static constexpr int kWavesCu = H == 32 && R >= 4 && !kHist ? kManyWavesCu : kMaxWavesCu;
+  static constexpr int kByWaves = kWavesCu / (R * S) > 0 ? kWavesCu / (R * S) : 1;
   static constexpr int kCtasPerCu = kByLds < kByWaves ? kByLds : kByWaves;
   static constexpr int kThreads = R * S * kWave;
   static constexpr int kWavesPerSimd = (kCtasPerCu * R * S + 3) / 4;
@@ -276,10 +281,10 @@ __device__ __forceinline__ void wait_vmcnt(int n) {
 // kMask = false: a.mask is null (prefill), known at compile time, so the page loop carries no
 // mask state.
 template <int H, int R, bool kHist, bool kMask>
-__global__ __launch_bounds__((Shape<R, kHist>::kThreads)) __attribute__((amdgpu_waves_per_eu(
-    Shape<R, kHist>::kWavesPerSimd))) void mqa_logits_decode_kernel(const DecodeArgs a) {
+__global__ __launch_bounds__((Shape<H, R, kHist>::kThreads)) __attribute__((amdgpu_waves_per_eu(
+    Shape<H, R, kHist>::kWavesPerSimd))) void mqa_logits_decode_kernel(const DecodeArgs a) {
   constexpr int HT = H / 16;  // head tiles
-  using Sh = Shape<R, kHist>;
+  using Sh = Shape<H, R, kHist>;
   constexpr int S = Sh::S;
   constexpr int NS = Sh::NS;
   static_assert(NS == 2 || NS == 3, "2 or 3 page slots per stream");
@@ -599,12 +604,12 @@ template <int H, int R, bool kHist>
 void launch_one(const DecodeArgs& a, uint32_t grid, hipStream_t stream) {
   if constexpr (R == 8) {  // eight rows a CTA: the prefill shape, which writes no mask
     if (a.mask == nullptr) {
-      hipLaunchKernelGGL((mqa_logits_decode_kernel<H, R, kHist, false>), dim3(grid), dim3(Shape<R, kHist>::kThreads),
+      hipLaunchKernelGGL((mqa_logits_decode_kernel<H, R, kHist, false>), dim3(grid), dim3(Shape<H, R, kHist>::kThreads),
                          0, stream, a);
       return;
     }
   }
-  hipLaunchKernelGGL((mqa_logits_decode_kernel<H, R, kHist, true>), dim3(grid), dim3(Shape<R, kHist>::kThreads), 0,
+  hipLaunchKernelGGL((mqa_logits_decode_kernel<H, R, kHist, true>), dim3(grid), dim3(Shape<H, R, kHist>::kThreads), 0,
                      stream, a);
 }
 
@@ -617,6 +622,9 @@ void launch_r(const DecodeArgs& a, int R, uint32_t grid, hipStream_t stream) {
     case 4:
       if constexpr (!kHist) launch_one<H, 4, false>(a, grid, stream);
       break;
+    case 6:
+      if constexpr (!kHist) launch_one<H, 6, false>(a, grid, stream);
+      break;
     default:
       if constexpr (!kHist) launch_one<H, 8, false>(a, grid, stream);
       break;
@@ -624,17 +632,37 @@ void launch_r(const DecodeArgs& a, int R, uint32_t grid, hipStream_t stream) {
 }
 
 // (CTAs per CU, pages per CTA) of a launch shape, on the host.
-void shape_host(int R, bool hist, int& ctas_per_cu, int& max_pages) {
-  switch (hist ? R + 16 : R) {
-    case 1: ctas_per_cu = Shape<1, false>::kCtasPerCu; max_pages = Shape<1, false>::kMaxPages; break;
-    case 2: ctas_per_cu = Shape<2, false>::kCtasPerCu; max_pages = Shape<2, false>::kMaxPages; break;
-    case 3: ctas_per_cu = Shape<3, false>::kCtasPerCu; max_pages = Shape<3, false>::kMaxPages; break;
-    case 4: ctas_per_cu = Shape<4, false>::kCtasPerCu; max_pages = Shape<4, false>::kMaxPages; break;
-    case 8: ctas_per_cu = Shape<8, false>::kCtasPerCu; max_pages = Shape<8, false>::kMaxPages; break;
-    case 17: ctas_per_cu = Shape<1, true>::kCtasPerCu; max_pages = Shape<1, true>::kMaxPages; break;
-    case 18: ctas_per_cu = Shape<2, true>::kCtasPerCu; max_pages = Shape<2, true>::kMaxPages; break;
-    default: ctas_per_cu = Shape<3, true>::kCtasPerCu; max_pages = Shape<3, true>::kMaxPages; break;
+template <int H, bool kHist>
+void shape_host(int R, int& ctas_per_cu, int& max_pages) {
+  auto of = [&](auto shape) {
+    ctas_per_cu = decltype(shape)::kCtasPerCu;
+    max_pages = decltype(shape)::kMaxPages;
+  };
+  switch (R) {
+    case 1: of(Shape<H, 1, kHist>{}); break;
+    case 2: of(Shape<H, 2, kHist>{}); break;
+    case 3: of(Shape<H, 3, kHist>{}); break;
+    case 4: of(Shape<H, 4, false>{}); break;
+    case 6: of(Shape<H, 6, false>{}); break;
+    default: of(Shape<H, 8, false>{}); break;
   }
+}
+
+// Rows per CTA when the caller leaves it open: a K page is read once per CTA row-set, so a group of
+// 4, 6 or 8 rows (or a multiple) takes one of that many rows.  Measured against two rows (us a launch;
+// requests x rows, tokens): 32 heads 8 x 6, 73,000 40.5 -> 24.7; 32 x 6, 8K-30K 39.7 -> 24.6; 64 x 4, 2K-50K
+// 67.9 -> 57.9; 16 x 8, 20K-60K 45.2 -> 30.2; 64 heads 64 x 4, 2K-50K 79.7 -> 68.5; 16 x 8, 20K-60K 53.9 ->
+// 46.5; 8 x 6, 16K-131K 37.5 -> 35.0 with three rows (35.7 with six: there the matrix work bounds both,
+// and a three-row CTA's shorter barriers win).  With few pages the launch is one latency chain and more,
+// smaller CTAs win (1 x 6 rows of 16,384 tokens, 256 pages: 5.1 with two rows, 5.7 with six; 2 x 4 of 4000:
+// 4.3 / 4.7; 4 x 4 of 30,000, 1876 pages: 12.8 / 11.5): four pages a CU is the line.
+int auto_rows(int heads, int group, int64_t batch, int64_t bt_pages, int64_t n_cu) {
+  const int few = group % 2 == 0 ? 2 : 1;
+  if (batch / group * bt_pages < 4 * n_cu) return few;
+  if (group % 8 == 0) return 8;
+  if (group % 6 == 0) return heads == 32 ? 6 : 3;
+  if (group % 4 == 0) return 4;
+  return few;
 }
 
 // Pages of the slices a prefill launch of n_groups 8-row groups cuts its width_pages K pages into
@@ -668,7 +696,10 @@ int enqueue(DecodeArgs a, int heads, int R, int target_ctas, bool hist, const in
   const int64_t n_groups = a.batch / R;
   DSA_REQUIRE(n_groups <= 0x3FFFFFFF, "%s: too many rows", who);
   int ctas_per_cu = 1, max_cta_pages = 1;
-  shape_host(R, hist, ctas_per_cu, max_cta_pages);
+  if (heads == 64 && hist) shape_host<64, true>(R, ctas_per_cu, max_cta_pages);
+  else if (heads == 64) shape_host<64, false>(R, ctas_per_cu, max_cta_pages);
+  else if (hist) shape_host<32, true>(R, ctas_per_cu, max_cta_pages);
+  else shape_host<32, false>(R, ctas_per_cu, max_cta_pages);
   a.slice_pages = 0;
   if (target_ctas <= 0) {
     // All CTAs resident at once: the per-group rounding adds up to one CTA per group, so aim
@@ -723,8 +754,8 @@ int enqueue(DecodeArgs a, int heads, int R, int target_ctas, bool hist, const in
 int enqueue_slices(DecodeArgs a, int heads, hipStream_t stream, const char* who) {
   constexpr int R = 8;
   const int64_t n_groups = (a.batch + R - 1) / R;
-  int ctas_per_cu = 1, max_cta_pages = 1, n_cu = 0;
-  shape_host(R, false, ctas_per_cu, max_cta_pages);
+  constexpr int max_cta_pages = Shape<64, R, false>::kMaxPages;
+  int n_cu = 0;
   const int st = dsa_device_cu_count(&n_cu);
   if (st != DSA_OK) return st;
   const int64_t width_pages = (a.width + kPage - 1) / kPage;
@@ -755,7 +786,8 @@ extern "C" int dsa_mqa_logits_decode(const uint8_t* q8, const float* w, int head
   DSA_REQUIRE(heads == 32 || heads == 64, "dsa_mqa_logits_decode: heads must be 32 or 64 (got %d)", heads);
   DSA_REQUIRE(batch >= 0 && group_size >= 1, "dsa_mqa_logits_decode: batch must be >= 0 and group_size >= 1");
   DSA_REQUIRE(batch % group_size == 0, "dsa_mqa_logits_decode: batch must be a multiple of group_size");
-  if (rows_per_cta <= 0) rows_per_cta = group_size % 2 == 0 ? 2 : 1;
+  const bool open = rows_per_cta <= 0;  // replaced below, once the sizes are checked
+  if (open) rows_per_cta = group_size % 2 == 0 ? 2 : 1;
   DSA_REQUIRE((rows_per_cta >= 1 && rows_per_cta <= 4 || rows_per_cta == 8) && group_size % rows_per_cta == 0,
               "dsa_mqa_logits_decode: rows_per_cta must be 1, 2, 3, 4 or 8 and divide group_size");
   DSA_REQUIRE(bt_pages > 0 && bt_pages * kPage <= 0x7FFFFFFF,
@@ -777,6 +809,14 @@ extern "C" int dsa_mqa_logits_decode(const uint8_t* q8, const float* w, int head
   const bool hist = fuse_pass1 != 0;
   DSA_REQUIRE(!hist || rows_per_cta <= 3,
               "dsa_mqa_logits_decode: the fused histogram needs rows_per_cta <= 3 (8 KB of LDS per row)");
+
+  // a caller's own CTA count or a fused histogram (at most three rows) keeps the two-row CTAs
+  if (open && !hist && target_ctas <= 0) {
+    int n_cu = 0;
+    const int st = dsa_device_cu_count(&n_cu);
+    if (st != DSA_OK) return st;
+    rows_per_cta = auto_rows(heads, group_size, batch, bt_pages, n_cu);
+  }
 
   DecodeArgs a{};
   a.q8 = q8;

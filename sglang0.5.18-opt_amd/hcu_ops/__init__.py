@@ -26,7 +26,8 @@ _TOPK_SPLITS = int(os.environ.get("HCU_TOPK_SPLITS", "8"))
 #   HCU_MQA_PCTAS[_G1]   CTAs per request row-set for grouped [single] rows; <= 0 takes every CTA that
 #                        is resident at once (on gfx950 that beats the reference's -1 policy of 64 per
 #                        row-set for few rows: the balanced grid spreads the pages over the whole chip).
-#   HCU_MQA_RPC          rows of a group sharing one K page stream (must divide the group).
+#   HCU_MQA_RPC          rows of a group sharing one K page stream (must divide the group).  Not set, an
+#                        even group takes as many as its sizes make fastest (up to eight).
 #   HCU_MQA_HIST_MAX_ROWS[_G6]  up to this many single [grouped] rows, when the paired top-k will split
 #                        rows, mqa_logits(..., hist_lens) builds the top-k's pass-1 histogram inside the
 #                        logits kernel (rows_per_cta <= 3).
@@ -43,6 +44,7 @@ _TOPK_SPLITS = int(os.environ.get("HCU_TOPK_SPLITS", "8"))
 _MQA_PCTAS = int(os.environ.get("HCU_MQA_PCTAS", "0"))
 _MQA_PCTAS_G1 = int(os.environ.get("HCU_MQA_PCTAS_G1", str(_MQA_PCTAS)))
 _MQA_RPC = int(os.environ.get("HCU_MQA_RPC", "2"))
+_MQA_RPC_OPEN = "HCU_MQA_RPC" not in os.environ
 _MQA_HIST_MAX_ROWS = int(os.environ.get("HCU_MQA_HIST_MAX_ROWS", "0"))
 _MQA_HIST_MAX_ROWS_G6 = int(os.environ.get("HCU_MQA_HIST_MAX_ROWS_G6", "0"))
 _MQA_PAIR_MAX_ROWS = int(os.environ.get("HCU_MQA_PAIR_MAX_ROWS", "256"))
@@ -135,6 +137,8 @@ def mqa_logits(q, kv_cache, weights, context_lens, block_table, max_context_len,
         persistent_ctas = _MQA_PCTAS_G1 if group_size == 1 else _MQA_PCTAS
     if rows_per_cta is None:
         rows_per_cta = 1 if group_size == 1 else _MQA_RPC
+        if _MQA_RPC_OPEN and rows_per_cta == 2 and group_size % 2 == 0:
+            rows_per_cta = 0  # chosen by the library
     hist_max_rows = _MQA_HIST_MAX_ROWS if group_size == 1 else _MQA_HIST_MAX_ROWS_G6
     use_hist = (hist_lens is not None and _TOPK_IMPL == "split"
                 and rows <= max(hist_max_rows, _MQA_PAIR_MAX_ROWS)
