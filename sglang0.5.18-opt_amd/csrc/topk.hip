@@ -7,8 +7,9 @@
 // order, then the ties taken in ascending token order -- a function of the scores alone, so
 // the layout is the same on every run and every graph replay.
 //
-// Algorithm (this file's own).  Default path, one read of the row: a fixed sample of the row
-// (256 chunks of 16 tokens, or the whole row up to 4096 tokens) gives a key K* that leaves, with
+// Algorithm (this file's own).  Rows of up to 8192 tokens are held in registers and their threshold
+// found by counting (held_row).  Longer rows, one read of the row: a fixed sample of the row
+// (256 chunks of 16 tokens) gives a key K* that leaves, with
 // overwhelming probability, between 2048 and a few thousand of the row's keys >= K*; one
 // unordered pass collects them (positions from wave-aggregated LDS atomics, no barriers in the
 // streaming loop); they are resolved exactly by a 12-bit histogram of a digit relative to K*
@@ -33,6 +34,7 @@
 // Many rows: one CTA per row does everything.  No host synchronisation; launch shapes depend
 // only on (rows, width, splits), so the whole path can be captured in a hipGraph.
 #include <mutex>
+#include <type_traits>
 
 #include "dsa_common.h"
 
@@ -47,7 +49,6 @@ constexpr int kCapW = 5120; // the same for the one-CTA-per-row kernel on scores
 constexpr int kWideRow = 81920;
 constexpr int kMaxSplit = 64;
 constexpr int64_t kMaxWidth = int64_t{1} << 29;  // tokens a row may hold: byte offsets stay below 2^31
-constexpr int kRankDirect = 128;  // members of the threshold digit ranked pairwise; more take radix passes
 constexpr int kUnroll = 4;  // float4 groups per lane in one batch (two batches in flight)
 
 struct RowSrc {
@@ -451,8 +452,8 @@ __device__ __forceinline__ void collect_bin(const RowSrc& rr, int b, int n_batch
 // resolved exactly among them; when the count misses that window the row takes the exact
 // two-pass path instead, so the result never depends on the sample.
 //
-// Sample: 256 chunks of 16 aligned tokens spread evenly over the row (one 64-B sector of
-// scores and one mask word each), or the whole row when it has <= 4096 tokens.  K* is the lower
+// Sample: 256 chunks of 16 aligned tokens spread evenly over a row of more than 4096 tokens (one 64-B
+// sector of scores and one mask word each).  K* is the lower
 // edge of the 4096-key digit (key[31:12]) holding the sample key of rank k (descending), k =
 // mu + 4 sqrt(mu) + 2, mu = 2048 * 4096 / len the expected number of sample keys above the row's
 // 2048th key: the row has fewer than 2048 keys >= K* only if the sample holds >= k keys above
@@ -462,7 +463,6 @@ constexpr int kSampleChunks = 256;
 constexpr int kSample = kSampleChunks * 16;
 
 __device__ __forceinline__ int sample_rank(int len) {
-  if (len <= kSample) return kTopK;  // the sample is the row: K* is its 2048th key
   const float mu = static_cast<float>(kTopK) * static_cast<float>(kSample) / static_cast<float>(len);
   const int k = static_cast<int>(ceilf(mu + 4.0f * sqrtf(mu) + 2.0f));
   return k < kSample ? k : kSample;
@@ -470,14 +470,12 @@ __device__ __forceinline__ int sample_rank(int len) {
 
 // Rank of the sample key that estimates the row's 2048th key (mu, rounded).
 __device__ __forceinline__ int sample_mid_rank(int len) {
-  if (len <= kSample) return kTopK;
   const int m = static_cast<int>(static_cast<float>(kTopK) * static_cast<float>(kSample) / static_cast<float>(len) + 0.5f);
   return m < 1 ? 1 : m;
 }
 
 // First token of sample quad s (4 tokens) of a row.
 __device__ __forceinline__ int sample_quad(int len, int s) {
-  if (len <= kSample) return s * 4;
   const int c = s >> 2;
   int start = static_cast<int>((static_cast<int64_t>(2 * c + 1) * len) / (2 * kSampleChunks)) & ~15;
   const int last = (len - 16) & ~15;
@@ -1017,15 +1015,13 @@ __device__ __forceinline__ int sparse_fast_case(int n_pos, const SampleCut& cut)
 // taken, its members are ranked exactly by (key desc, token asc) -- a handful by the choice of
 // the digit -- which also gives the threshold key; the taken tokens then go out in order
 // (emit_held).  More members than threads (heavy ties) select the threshold by radix passes
-// and emit by re-reading the row r.  kShort: the candidates are a whole short row cut at 0 on
-// key[31:20]; there, more than kRankDirect members take two radix passes instead of the ranking
-// (measured on 64 rows of 4096 tokens with 300 / 512 members: 23.2 / 32.9 us -> 9.9 us).
+// and emit by re-reading the row r.
 // Returns false, having written nothing, when the row's positive keys must be counted exactly
 // first (sparse_fast_case): the caller runs exact_row.
 // kGivenPv: load(e, key, token, entry) also hands over each candidate's page-table entry
 // (gathered by the CTA that collected it); otherwise load(e, key, token) and the entries are
 // gathered here.
-template <bool kVec, bool kShort, bool kGivenPv = false, int NT, int CAP, typename Load>
+template <bool kVec, bool kGivenPv = false, int NT, int CAP, typename Load>
 __device__ __forceinline__ bool resolve_cands(ResolveLds<NT, CAP>& L, int n, const SampleCut& cut, const RowSrc& r, const PtRow& pt,
                               int32_t* dst, Load load) {
   constexpr int EPT = CAP / NT;
@@ -1129,35 +1125,7 @@ __device__ __forceinline__ bool resolve_cands(ResolveLds<NT, CAP>& L, int n, con
   __syncthreads();
   bool take = false, tie = false;
   int tok = 0, val = 0;
-  if (kShort && n_t1 > kRankDirect && !plus0) {  // block-uniform
-    // Many members of one plain 12-bit digit (a short row, resolved whole on key[31:20] = t1), at
-    // most one per thread: the threshold key by two 1024-bin passes over key[19:10] and key[9:0]
-    // in L.ck (free now) instead of ranking each member against all the others.  Every member at
-    // the threshold is flagged a tie and the tie count is the ties to take: the ordered emission
-    // gives them the last slots in token order and drops the rest.
-    int* ha = reinterpret_cast<int*>(L.ck);
-    int* hb = ha + 1024;
-    zero_lds<NT>(ha, 2048);
-    uint32_t k = 0u;
-    if (tid < n_t1) {
-      k = mk[tid];
-      tok = mt[tid];
-      val = mv[tid];
-    }
-    __syncthreads();
-    if (tid < n_t1) atomicAdd(&ha[(k >> 10) & 1023u], 1);
-    __syncthreads();
-    find_threshold<1024, NT>(ha, need1, L.wtot, L.res);
-    const uint32_t da = static_cast<uint32_t>(L.res[0]);
-    const int above_a = L.res[1];
-    if (tid < n_t1 && ((k >> 10) & 1023u) == da) atomicAdd(&hb[k & 1023u], 1);
-    __syncthreads();
-    find_threshold<1024, NT>(hb, need1 - above_a, L.wtot, L.res);
-    const uint32_t thr = (t1 << 20) | (da << 10) | static_cast<uint32_t>(L.res[0]);
-    take = tid < n_t1 && k >= thr;
-    tie = tid < n_t1 && k == thr;
-    if (tid == 0) L.misc[3] = need1 - above_a - L.res[1];  // read by emit_held after its first barrier
-  } else {
+  {
     // A member is taken when its (key desc, token asc) rank is below need1; it is a tie when the
     // members with a key >= its own reach need1, i.e. its key is the threshold (the need1-th).
     // With exactly 2048 positive keys the reference's threshold is +0 and nothing is a tie.
@@ -1215,35 +1183,346 @@ __device__ __forceinline__ bool resolve_cands(ResolveLds<NT, CAP>& L, int n, con
   return true;
 }
 
-// A row of at most kSample tokens: every key goes to the candidate list at its token's
-// position (no threshold, no collection pass) and is resolved on the plain 12-bit digit.
-template <bool kVec, int NT, int CAP>
-__device__ __forceinline__ bool small_row(ResolveLds<NT, CAP>& L, const RowSrc& r, const PtRow& pt, int32_t* dst) {
-  static_assert(CAP >= kSample, "the row fits the candidate list");
-  constexpr int QPT = kSample / 4 / NT;
+// ---------------------------------------------------------------------------------------------
+// Rows of up to NT * 4 * Q tokens held in registers, one CTA a row, exact whatever the scores: no
+// sample, no candidate list, no fallback and no LDS histogram.  The 2048th largest key is found by
+// counting: a round counts the keys >= a probe (one compare and one ballot's popcount a key, one barrier
+// for the waves' counts), and the probes close in on it until at most 64 keys are left between, which
+// every wave ranks for itself.  Probes: the smallest positive key (it settles the rows of the sparse fast
+// path in one or two rounds), the row's quantile if its scores were normal (mean and deviation come
+// with the first count), a step from there by the normal density, then interpolation of the counts
+// between the bracket's float values with the Illinois weights; four or five rounds on the indexer's
+// logits.  Every third round from the sixth pulls the bracket's ends in to keys of the row, which ends
+// the search on heavy ties, and past kHeldGuess rounds the probes halve the key range, so that no input
+// takes more than 32 further ones.
+constexpr int kHeldGuess = 18;
+constexpr int kHeldQ = 4;                      // quads a thread of the kTs-thread kernels
+constexpr int kHeldRow = kTs * 4 * kHeldQ;     // rows of up to this many tokens are held
+
+__device__ __forceinline__ float key_value(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k ^ 0x80000000u) : ~k);
+}
+
+// max / min over the wave, in every lane (16-lane rows by DPP, then the rows' first lanes)
+template <bool kMax>
+__device__ __forceinline__ uint32_t wave_extreme(uint32_t x) {
+  auto pick = [](uint32_t p, uint32_t q) { return kMax ? max(p, q) : min(p, q); };
+  x = pick(x, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0xB1, 0xF, 0xF, false)));
+  x = pick(x, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x4E, 0xF, 0xF, false)));
+  x = pick(x, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x141, 0xF, 0xF, false)));
+  x = pick(x, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x140, 0xF, 0xF, false)));
+  auto at = [&](int l) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), l)); };
+  return pick(pick(at(0), at(16)), pick(at(32), at(48)));
+}
+
+__device__ __forceinline__ float wave_total(float x) {
+  auto dpp = [](float y, auto c) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(y), decltype(c)::value, 0xF, 0xF, false));
+  };
+  x += dpp(x, std::integral_constant<int, 0xB1>{});
+  x += dpp(x, std::integral_constant<int, 0x4E>{});
+  x += dpp(x, std::integral_constant<int, 0x141>{});
+  x += dpp(x, std::integral_constant<int, 0x140>{});
+  auto at = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l)); };
+  return (at(0) + at(16)) + (at(32) + at(48));
+}
+
+// z with P(normal > z) = q (Abramowitz and Stegun 26.2.23, |error| < 4.5e-4).
+__device__ __forceinline__ float normal_quantile(float q) {
+  const float t = sqrtf(-2.0f * __logf(fminf(q, 1.0f - q)));
+  const float z = t - (2.515517f + t * (0.802853f + t * 0.010328f)) /
+                          (1.0f + t * (1.432788f + t * (0.189269f + t * 0.001308f)));
+  return q <= 0.5f ? z : -z;
+}
+
+template <int NT, int Q>
+struct alignas(16) HeldLds {
+  int cnt[2][NT / kWave];
+  uint32_t top[NT / kWave];
+  uint32_t low[NT / kWave];
+  float sum[NT / kWave];
+  float sq[NT / kWave];
+  uint32_t tot[Q * (NT / kWave)];
+  uint32_t mem[kWave];
+  int n_mem;
+  uint16_t out[kTopK + kWave];  // the selected tokens in output order; then a discard word a lane
+};
+
+template <bool kVec, int NT, int Q>
+__device__ __forceinline__ void held_row(HeldLds<NT, Q>& L, const RowSrc& r, const PtRow& pt, int32_t* dst) {
+  constexpr int W = NT / kWave;
+  constexpr int QW = Q * W;
+  static_assert(W % 4 == 0 && QW <= 2 * kWave, "counts read 16 B at a time; two totals a lane at most");
+  static_assert(NT * 4 * Q <= 65536 && kTopK % NT == 0, "16-bit tokens; the output split over the block");
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int len = r.len;
+  // Quad u of thread tid: tokens 4 (u NT + tid) ..; tokens past the row get key 0, which only ties
+  // with real tokens before them, and a row has more than 2048 of those.
+  uint32_t k[Q][4];
+  float sum = 0.0f, sq = 0.0f;
+  {
+    Quad q[Q];
 #pragma unroll
-  for (int j = 0; j < QPT; ++j) {
-    const int i0 = (static_cast<int>(threadIdx.x) + j * NT) * 4;
-    Quad q;
-    load_quad<kVec>(r, i0, q);
-    uint32_t k[4];
-    const uint32_t v = quad_keys(r, i0, q, k);
+    for (int u = 0; u < Q; ++u) load_quad<kVec>(r, (u * NT + tid) * 4, q[u]);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if ((v >> e) & 1u) {
-        L.ck[i0 + e] = k[e];
-        L.ci[i0 + e] = i0 + e;
+    for (int u = 0; u < Q; ++u) {
+      const uint32_t live = quad_keys(r, (u * NT + tid) * 4, q[u], k[u]);
+      if ((u + 1) * NT * 4 > len) {  // block-uniform: the quads the row ends in
+#pragma unroll
+        for (int j = 0; j < 4; ++j) k[u][j] = (live >> j) & 1u ? k[u][j] : 0u;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float x = k[u][j] ? key_value(k[u][j]) : 0.0f;
+        sum += x;
+        sq = fmaf(x, x, sq);
+      }
+    }
+  }
+  // The row's keys >= key; every thread gets the sum.  parity alternates over the calls: a wave may
+  // write its next count while another still reads this one, not the one after.
+  int parity = 0;
+  auto count_ge = [&](uint32_t key) {
+    int c = 0;
+#pragma unroll
+    for (int u = 0; u < Q; ++u) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c += __popcll(__ballot(k[u][j] >= key));
+    }
+    if (lane == 0) L.cnt[parity][w] = c;
+    __syncthreads();
+    int n = 0;
+#pragma unroll
+    for (int v = 0; v < W / 4; ++v) {
+      const int4 x = reinterpret_cast<const int4*>(L.cnt[parity])[v];
+      n += x.x + x.y + x.z + x.w;
+    }
+    parity ^= 1;
+    return uniform(n);
+  };
+  // Pulls lo > 0 up and hi down to the nearest keys of the row (a count follows before the next call).
+  auto ends = [&](uint32_t& lo, uint32_t& hi) {
+    uint32_t m = 0xFFFFFFFFu, t = 0u;
+#pragma unroll
+    for (int u = 0; u < Q; ++u) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        m = min(m, k[u][j] >= lo ? k[u][j] : 0xFFFFFFFFu);
+        t = max(t, k[u][j] <= hi ? k[u][j] : 0u);
+      }
+    }
+    m = wave_extreme<false>(m);
+    t = wave_extreme<true>(t);
+    if (lane == 0) {
+      L.low[w] = m;
+      L.top[w] = t;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < W / 4; ++v) {
+      const uint4 x = reinterpret_cast<const uint4*>(L.top)[v];
+      const uint4 y = reinterpret_cast<const uint4*>(L.low)[v];
+      t = max(max(max(t, x.x), max(x.y, x.z)), x.w);
+      m = min(min(min(m, y.x), min(y.y, y.z)), y.w);
+    }
+    lo = static_cast<uint32_t>(uniform(static_cast<int>(m)));
+    hi = static_cast<uint32_t>(uniform(static_cast<int>(t)));
+  };
+  sum = wave_total(sum);
+  sq = wave_total(sq);
+  if (lane == 0) {
+    L.sum[w] = sum;
+    L.sq[w] = sq;
+    if (w == 0) L.n_mem = 0;
+  }
+  const int n_pos = count_ge(kZeroKey + 1u);
+
+  // thr: the 2048th largest key (+0 with no ties when the row holds exactly 2048 positive keys, the
+  // reference's sparse fast path, sparse_mask_topk.cu:199-234).  It lies in [lo, hi]; c_lo keys are
+  // >= lo, c_hi are > hi.
+  uint32_t thr = kZeroKey;
+  if (n_pos != kTopK) {  // block-uniform, like everything below
+    sum = sq = 0.0f;
+#pragma unroll
+    for (int v = 0; v < W / 4; ++v) {
+      const float4 f = reinterpret_cast<const float4*>(L.sum)[v];
+      const float4 g = reinterpret_cast<const float4*>(L.sq)[v];
+      sum += (f.x + f.y) + (f.z + f.w);
+      sq += (g.x + g.y) + (g.z + g.w);
+    }
+    uint32_t lo = 0u, hi = 0xFFFFFFFFu;
+    int c_lo = len, c_hi = 0;
+    if (n_pos > kTopK) {
+      lo = kZeroKey + 1u;
+      c_lo = n_pos;
+    } else {
+      hi = kZeroKey;
+      c_hi = n_pos;
+    }
+    float w_lo = static_cast<float>(c_lo - kTopK), w_hi = static_cast<float>(kTopK - c_hi);
+    const float inv_n = __builtin_amdgcn_rcpf(static_cast<float>(len));
+    const float mean = sum * inv_n;
+    const float dev = __builtin_amdgcn_sqrtf(fmaxf(sq * inv_n - mean * mean, 0.0f));
+    const float z = normal_quantile(static_cast<float>(kTopK) * inv_n);
+    float next = mean + z * dev;  // the next probe's value, for the first two rounds
+    int side = 0;
+    bool at_zero = n_pos < kTopK;  // first +0 itself: with its ties it may hold the 2048th
+    int round = 0;
+    while (lo < hi && c_lo - c_hi > kWave) {
+      uint32_t p;  // a probe in (lo, hi]
+      if (at_zero) {
+        p = hi;
+      } else {
+        p = float_key(next);
+        if (round >= 2 || !(p > lo && p <= hi)) {
+          if (lo == 0u || hi == 0xFFFFFFFFu || (round >= 6 && round % 3 == 0)) {
+            if (lo == 0u) {  // off key 0, which the tokens past the row hold
+              const int c = count_ge(1u);
+              if (c < kTopK) break;  // the 2048th is a key 0 of the row's own
+              lo = 1u;
+              c_lo = c;
+            }
+            ends(lo, hi);
+            if (lo == hi) break;
+          }
+          const float fl = key_value(lo), fh = key_value(hi);
+          // aimed a few keys to the near side of the 2048th, to bring the farther end close
+          const float aim = c_lo - c_hi <= 48 ? 0.0f : (c_lo - kTopK > kTopK - c_hi ? 12.0f : -12.0f);
+          const float f = (w_lo - aim) * __builtin_amdgcn_rcpf(w_lo + w_hi);
+          p = float_key(fl + (fh - fl) * fminf(fmaxf(f, 0.02f), 0.98f));
+          p = p > lo ? p : lo + 1u;
+          p = p < hi ? p : hi;
+          if (round >= kHeldGuess) p = lo + (hi - lo + 1u) / 2u;
+        }
+        ++round;
+      }
+      p = static_cast<uint32_t>(uniform(static_cast<int>(p)));
+      const int c = count_ge(p);
+      // a step past the quantile by the normal density there, so that the two probes bracket it
+      if (!at_zero && round == 1) {
+        const float off = static_cast<float>(c - kTopK) * 1.2f + (c >= kTopK ? 20.0f : -20.0f);
+        next = key_value(p) + off * 2.5066283f * dev * inv_n * __expf(0.5f * z * z);
+      }
+      at_zero = false;
+      if (c >= kTopK) {
+        lo = p;
+        c_lo = c;
+        w_lo = static_cast<float>(c - kTopK) + 0.5f;
+        if (side > 0) w_hi *= 0.5f;
+        side = 1;
+      } else {
+        hi = p - 1u;
+        c_hi = c;
+        w_hi = static_cast<float>(kTopK - c);
+        if (side < 0) w_lo *= 0.5f;
+        side = -1;
+      }
+    }
+    thr = lo;
+    if (lo < hi && c_lo - c_hi <= kWave) {  // the 2048th is among the at most 64 keys in [lo, hi]
+      // those above 0 (tokens past the row hold key 0); fewer of them than needed: it is a key 0
+      const uint32_t from = lo > 0u ? lo : 1u;
+      const uint32_t span = hi - from;
+#pragma unroll
+      for (int u = 0; u < Q; ++u) {
+        if (min(min(k[u][0] - from, k[u][1] - from), min(k[u][2] - from, k[u][3] - from)) <= span) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if (k[u][j] - from <= span) {
+              const int at = atomicAdd(&L.n_mem, 1);
+              if (at < kWave) L.mem[at] = k[u][j];
+            }
+          }
+        }
+      }
+      __syncthreads();
+      const int m = uniform(min(L.n_mem, kWave));
+      const int need = kTopK - c_hi;
+      const uint32_t km = L.mem[lane];
+      int gt = 0, ge = 0;
+      for (int j = 0; j < m; ++j) {
+        const uint32_t kj = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(km), j));
+        gt += kj > km;
+        ge += kj >= km;
+      }
+      const uint64_t hit = __ballot(lane < m && gt < need && need <= ge);
+      if (hit) thr = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(km), __builtin_ctzll(hit)));
+    }
+  }
+
+  // Ordered emission: above the threshold in token order, then the ties.  A (quad, wave)'s counts travel
+  // in one word (ties in the upper half); their prefix in token order, which every wave forms for
+  // itself, places the selected tokens in LDS, and the block writes the row from there: one coalesced
+  // store and one page-table gather per output entry.
+  int before[Q];  // tokens above the threshold in the lower lanes' part of the quad row
+#pragma unroll
+  for (int u = 0; u < Q; ++u) {
+    int b4 = 0, n_gt = 0, n_eq = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint64_t m = __ballot(k[u][j] > thr);
+      b4 = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+          static_cast<uint32_t>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), static_cast<uint32_t>(b4))));
+      n_gt += __popcll(m);
+      n_eq += __popcll(__ballot(k[u][j] == thr));
+    }
+    before[u] = b4;
+    if (lane == 0) L.tot[u * W + w] = static_cast<uint32_t>(n_gt) | (static_cast<uint32_t>(n_eq) << 16);
+  }
+  __syncthreads();
+  const uint32_t t0 = lane < QW ? L.tot[lane] : 0u;
+  const uint32_t i0 = static_cast<uint32_t>(wave_prefix_sum(static_cast<int>(t0)));
+  uint32_t total = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(i0), 63));
+  uint32_t t1 = 0u, i1 = 0u;
+  if constexpr (QW > kWave) {
+    t1 = kWave + lane < QW ? L.tot[kWave + lane] : 0u;
+    i1 = total + static_cast<uint32_t>(wave_prefix_sum(static_cast<int>(t1)));
+    total = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(i1), 63));
+  }
+  const int base_t = static_cast<int>(total & 0xFFFFu);
+  const int trash = kTopK + lane;
+#pragma unroll
+  for (int u = 0; u < Q; ++u) {
+    const int at = u * W + w;  // wave-uniform
+    const bool second = QW > kWave && at >= kWave;
+    const uint32_t cw = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(second ? t1 : t0), at & 63));
+    if (cw == 0u) continue;  // wave-uniform: nothing selected here
+    const uint32_t b = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(second ? i1 : i0), at & 63)) - cw;
+    int pa = static_cast<int>(b & 0xFFFFu) + before[u];
+    const int tok = (u * NT + tid) * 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const bool above = k[u][j] > thr;
+      L.out[above ? pa : trash] = static_cast<uint16_t>(tok + j);
+      pa += above;
+    }
+    if (cw >> 16) {  // wave-uniform: ties among them, in (lane, j) order
+      int pq = base_t + static_cast<int>(b >> 16);
+      int e = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint64_t m = __ballot(k[u][j] == thr);
+        e = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+            static_cast<uint32_t>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), static_cast<uint32_t>(e))));
+      }
+      pq += e;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool tie = k[u][j] == thr;
+        L.out[tie ? min(pq, trash) : trash] = static_cast<uint16_t>(tok + j);
+        pq += tie;
       }
     }
   }
   __syncthreads();
-  SampleCut cut;
-  cut.thr = 0u;
-  cut.shift = 20;
-  return resolve_cands<kVec, true>(L, r.len, cut, r, pt, dst, [&](int e, uint32_t& k, int& t) {
-    k = L.ck[e];
-    t = L.ci[e];
-  });
+  constexpr int kPer = kTopK / NT;
+  int32_t e[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) e[j] = pt.at(L.out[tid + j * NT], true);
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) dst[tid + j * NT] = e[j];
 }
 
 struct TopkArgs {
@@ -1303,6 +1582,20 @@ __device__ __forceinline__ void copy_short_row(const PtRow& pt, int32_t* dst, in
 }
 
 // ---------------------------------------------------------------------------------------------
+// One CTA a row for scores of at most NT * 4 * Q tokens: all that held_row needs, so that eight waves
+// a SIMD hide each other's rounds.
+template <bool kVec, int NT, int Q>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void topk_held_kernel(const TopkArgs a) {
+  __shared__ HeldLds<NT, Q> L;
+  const int row = blockIdx.x;
+  const int len = row_len(a, row);
+  const PtRow pt = pt_row(a, row);
+  int32_t* dst = a.out + static_cast<int64_t>(row) * kTopK;
+  if (len <= kTopK) copy_short_row<NT>(pt, dst, len);
+  else held_row<kVec, NT, Q>(L, row_src(a, row, len), pt, dst);
+}
+
+// ---------------------------------------------------------------------------------------------
 // One CTA per row with pass 1 (histogram + counts) from a.ghist / a.gcnt (the logits kernel's
 // fused pass 1): the row's threshold from its exact threshold bin, then the ordered emission.
 template <bool kVec>
@@ -1358,7 +1651,12 @@ __global__ __launch_bounds__(kTk) void topk_single_kernel(const TopkArgs a) {
 template <bool kVec, int CAP>
 __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void topk_row_sampled_kernel(
     const TopkArgs a) {
-  __shared__ ResolveLds<kTs, CAP> L;
+  __shared__ union Lds {
+    ResolveLds<kTs, CAP> res;
+    HeldLds<kTs, kHeldQ> held;
+    __device__ Lds() {}
+  } lds;
+  ResolveLds<kTs, CAP>& L = lds.res;
   constexpr int kStep = kTs * 4 * kUnroll;
   const int row = blockIdx.x;
   const int len = row_len(a, row);
@@ -1369,12 +1667,12 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
     return;
   }
   const RowSrc r = row_src(a, row, len);
+  if (len <= kHeldRow) {  // block-uniform
+    held_row<kVec, kTs, kHeldQ>(lds.held, r, pt, dst);
+    return;
+  }
   bool done = false;
-  if (len <= kSample) {  // block-uniform
-    // unaligned rows (scalar loads) take the exact path: small_row beside it would push this
-    // variant past 128 VGPRs into scratch
-    if constexpr (kVec) done = small_row<kVec, kTs>(L, r, pt, dst);
-  } else {
+  {
     const int b0 = static_cast<int>(threadIdx.x) * 4;
     SampleLoads<kTs> smp;
     sample_issue<kVec, kTs>(r, smp);  // the sample first: it is needed first
@@ -1420,7 +1718,7 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
       n = L.misc[2];
     }
     if (n >= kTopK && n <= CAP) {  // block-uniform
-      done = resolve_cands<kVec, false>(L, n, cut, r, pt, dst, [&](int e, uint32_t& k, int& t) {
+      done = resolve_cands<kVec>(L, n, cut, r, pt, dst, [&](int e, uint32_t& k, int& t) {
         collected(L.ck[e], L.ci[e], k, t);
       });
     }
@@ -1476,6 +1774,7 @@ struct SampledLds {
       int ci[CAP + kWave];
     } col;                          // this CTA's keys >= K* (raw bits; discard words past CAP)
     ResolveLds<kTs, CAP> res;       // the threshold search; the row's resolution (last CTA)
+    HeldLds<kTs, kHeldQ> held;      // a short row
   } u;
   int wtot[kTs / kWave];
   int res[6];
@@ -1574,10 +1873,11 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
   // the row's scores stays live across the collection loop
   auto dst = [&]() { return a.out + static_cast<int64_t>(row) * kTopK; };
   bool done = false;
-  if (len <= kSample) {  // the whole row in one CTA, no split
-    if (slice != 0) return;
-    done = small_row<kVec, kTs>(L.u.res, r, pt_row(a, row), dst());
-  } else {
+  if (len <= kHeldRow) {  // the whole row in one CTA, no split
+    if (slice == 0) held_row<kVec, kTs, kHeldQ>(L.u.held, r, pt_row(a, row), dst());
+    return;
+  }
+  {
     int begin, end, n_sl;
     if (!split_slice(len, a.S, slice, begin, end, n_sl)) return;
     const RowSrc rr = row_src(a, row, end);
@@ -1649,7 +1949,7 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
 
     const int n_tot = L.n[3];
     if (n_tot >= kTopK && n_tot <= CAP) {  // block-uniform
-      done = resolve_cands<kVec, false, true>(L.u.res, n_tot, cut, r, pt_row(a, row), dst(),
+      done = resolve_cands<kVec, true>(L.u.res, n_tot, cut, r, pt_row(a, row), dst(),
                                               [&](int e, uint32_t& k, int& t, int32_t& v) {
         k = __hip_atomic_load(&lk[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         t = __hip_atomic_load(&lt[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1676,7 +1976,7 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
       __syncthreads();
       const int n2 = R.misc[2];
       if (n2 >= kTopK && n2 <= CAP) {  // block-uniform
-        done = resolve_cands<kVec, false>(R, n2, c2, r, pt_row(a, row), dst(), [&](int e, uint32_t& k, int& t) {
+        done = resolve_cands<kVec>(R, n2, c2, r, pt_row(a, row), dst(), [&](int e, uint32_t& k, int& t) {
           collected(R.ck[e], R.ci[e], k, t);
         });
       }
@@ -1810,6 +2110,13 @@ int resident_per_cu(Kernel kernel) {
   return n;
 }
 
+template <int NT, int Q>
+void launch_held(const TopkArgs& a, bool vec, hipStream_t stream) {
+  const dim3 grid(static_cast<uint32_t>(a.rows));
+  if (vec) hipLaunchKernelGGL((topk_held_kernel<true, NT, Q>), grid, dim3(NT), 0, stream, a);
+  else hipLaunchKernelGGL((topk_held_kernel<false, NT, Q>), grid, dim3(NT), 0, stream, a);
+}
+
 struct WsLayout {
   size_t ctr, c_keys, c_tok, c_pv, total;
 };
@@ -1895,10 +2202,19 @@ int topk_common(const float* score, int64_t score_stride, int64_t width, int64_t
       else hipLaunchKernelGGL((topk_single_kernel<false>), grid_rows, dim3(kTk), 0, stream, a);
     } else {
       const bool wide = cap_for(width) == kCapW;
-      if (vec && wide) hipLaunchKernelGGL((topk_row_sampled_kernel<true, kCapW>), grid_rows, dim3(kTs), 0, stream, a);
+      if (width <= kHeldRow) {
+        // Every row fits a CTA's registers (us a launch, sampled -> held: 4096 x 2049-4096 tokens 90.0 ->
+        // 38.0, 64 x 4096 13.7 -> 9.2, 1 x 4096 10.0 -> 6.7, 3904 x 4096-8000 123 -> 63, 32 x 8192 11.5 ->
+        // 10.6).  Up to 4096 tokens 512-thread CTAs while a CU has at most one, the shorter chain (1 x
+        // 4096: 6.7 against 8.0 with 256 threads; 250 rows 9.7 / 10.8), else 256 threads (1000 rows
+        // 16.7 -> 14.7, 4096 rows 48.3 -> 38.0).
+        if (width > 4096) launch_held<512, 4>(a, vec, stream);
+        else if (rows <= n_cu) launch_held<512, 2>(a, vec, stream);
+        else launch_held<256, 4>(a, vec, stream);
+      } else if (vec && wide) hipLaunchKernelGGL((topk_row_sampled_kernel<true, kCapW>), grid_rows, dim3(kTs), 0, stream, a);
       else if (vec) hipLaunchKernelGGL((topk_row_sampled_kernel<true, kCapS>), grid_rows, dim3(kTs), 0, stream, a);
-      else if (wide) hipLaunchKernelGGL((topk_row_sampled_kernel<false, kCapW>), grid_rows, dim3(kTs), 0, stream, a);
-      else hipLaunchKernelGGL((topk_row_sampled_kernel<false, kCapS>), grid_rows, dim3(kTs), 0, stream, a);
+      // unaligned rows always take the long list: its late page-table gather leaves room for the buffer loads
+      else hipLaunchKernelGGL((topk_row_sampled_kernel<false, kCapW>), grid_rows, dim3(kTs), 0, stream, a);
     }
     return check_launch(who);
   }
