@@ -49,11 +49,13 @@ void check_kv(const torch::Tensor& kv_cache) {
 // zws = [12-bit key histograms | zeros | (positives, zeros)] of the rows longer than 2048
 // (mqa_hist.cu:278-304); fuse_pass1 = false zeroes only the split top-k's per-row counters in
 // zws (the paired top-k then selects with its sampled threshold: no histogram is built).
-std::vector<torch::Tensor> mqa_logits_hist(const torch::Tensor& q, const torch::Tensor& kv_cache,
+// with_zws: zws is among the results even when there is no hist_lens (empty then).
+std::vector<torch::Tensor> mqa_logits_impl(const torch::Tensor& q, const torch::Tensor& kv_cache,
                                            const torch::Tensor& weights, const torch::Tensor& context_lens,
                                            const torch::Tensor& block_table, int64_t max_context_len,
                                            int64_t group_size, int64_t persistent_ctas, int64_t rows_per_cta,
-                                           const c10::optional<torch::Tensor>& hist_lens, bool fuse_pass1) {
+                                           const c10::optional<torch::Tensor>& hist_lens, bool fuse_pass1,
+                                           bool with_zws) {
   TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::kFloat8_e4m3fn && q.dim() == 4 && q.size(1) == 1 &&
                   (q.size(2) == 32 || q.size(2) == 64) && q.size(3) == kHeadDim && q.is_contiguous(),
               "q must be contiguous fp8 e4m3fn [B, 1, H, 128] with H in {32, 64}");
@@ -82,7 +84,8 @@ std::vector<torch::Tensor> mqa_logits_hist(const torch::Tensor& q, const torch::
   auto logits = torch::empty({B, max_context_len}, q.options().dtype(at::kFloat));
   const int64_t mask_stride = (max_context_len + 15) / 16;
   auto mask = torch::empty({B, mask_stride}, q.options().dtype(at::kShort));
-  auto zws = torch::empty({hist ? B * (2 * kBins + 2) : 0}, q.options().dtype(at::kInt));
+  torch::Tensor zws;
+  if (hist || with_zws) zws = torch::empty({hist ? B * (2 * kBins + 2) : 0}, q.options().dtype(at::kInt));
   const int64_t pages = block_table.size(1);
   const int64_t R = rows_per_cta > 0 ? rows_per_cta : (group_size % 2 == 0 ? 2 : 1);
   TORCH_CHECK(!(hist && fuse_pass1) || R <= 3,
@@ -96,7 +99,27 @@ std::vector<torch::Tensor> mqa_logits_hist(const torch::Tensor& q, const torch::
       mask.data_ptr<int16_t>(), mask_stride, rows_per_cta > 0 ? static_cast<int>(R) : 0, target,
       hist ? hist_lens->data_ptr<int>() : nullptr, hist ? zws.data_ptr<int>() : nullptr, hist && fuse_pass1 ? 1 : 0,
       cur_stream()));
+  if (!zws.defined()) return {logits, mask};
   return {logits, mask, zws};
+}
+
+std::vector<torch::Tensor> mqa_logits_hist(const torch::Tensor& q, const torch::Tensor& kv_cache,
+                                           const torch::Tensor& weights, const torch::Tensor& context_lens,
+                                           const torch::Tensor& block_table, int64_t max_context_len,
+                                           int64_t group_size, int64_t persistent_ctas, int64_t rows_per_cta,
+                                           const c10::optional<torch::Tensor>& hist_lens, bool fuse_pass1) {
+  return mqa_logits_impl(q, kv_cache, weights, context_lens, block_table, max_context_len, group_size,
+                         persistent_ctas, rows_per_cta, hist_lens, fuse_pass1, true);
+}
+
+// Logits and mask alone: no workspace tensor is made (an empty one costs 1.4 us of host time, as much as
+// a sixth of the call).
+std::vector<torch::Tensor> mqa_logits(const torch::Tensor& q, const torch::Tensor& kv_cache,
+                                      const torch::Tensor& weights, const torch::Tensor& context_lens,
+                                      const torch::Tensor& block_table, int64_t max_context_len, int64_t group_size,
+                                      int64_t persistent_ctas, int64_t rows_per_cta) {
+  return mqa_logits_impl(q, kv_cache, weights, context_lens, block_table, max_context_len, group_size,
+                         persistent_ctas, rows_per_cta, c10::nullopt, false, false);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -151,7 +174,8 @@ torch::Tensor topk_impl(const torch::Tensor& score, const c10::optional<torch::T
   const int cus = n_cu();
   const int splits = static_cast<int>(std::max<int64_t>(1, max_splits));
   const size_t ws_bytes = dsa_topk_workspace_bytes(rows, width, splits, cus);
-  auto ws = torch::empty({static_cast<int64_t>(ws_bytes)}, score.options().dtype(at::kByte));
+  torch::Tensor ws;  // only when rows are split
+  if (ws_bytes) ws = torch::empty({static_cast<int64_t>(ws_bytes)}, score.options().dtype(at::kByte));
   const int16_t* mp = nonzero_mask.has_value() ? nonzero_mask->data_ptr<int16_t>() : nullptr;
   const int64_t ms = nonzero_mask.has_value() ? nonzero_mask->stride(0) : 0;
   const int32_t* cu = decode_layout ? nullptr : cu_seqlens_q.data_ptr<int>();
@@ -419,6 +443,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("q"), py::arg("kv_cache"), py::arg("weights"), py::arg("context_lens"), py::arg("block_table"),
         py::arg("max_context_len"), py::arg("group_size"), py::arg("persistent_ctas"), py::arg("rows_per_cta"),
         py::arg("hist_lens"), py::arg("fuse_pass1") = true);
+  m.def("mqa_logits", &mqa_logits, "mqa_logits_hist without a paired top-k -> {logits, mask}", py::arg("q"),
+        py::arg("kv_cache"), py::arg("weights"), py::arg("context_lens"), py::arg("block_table"),
+        py::arg("max_context_len"), py::arg("group_size"), py::arg("persistent_ctas"), py::arg("rows_per_cta"));
   m.def("sparse_mask_topk_transform", &sparse_mask_topk_transform,
         "Exact top-2048 + page-table transform over sparse-mask MQA logits (one CTA per row)");
   m.def("sparse_mask_topk_transform_split", &sparse_mask_topk_transform_split,

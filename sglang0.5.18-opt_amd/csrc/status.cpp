@@ -1,6 +1,7 @@
 // Thread-local error status of the C ABI and small device queries.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <string>
@@ -39,9 +40,20 @@ int check_launch(const char* what) {
 extern "C" const char* dsa_last_error(void) { return g_last_error.c_str(); }
 
 extern "C" int dsa_device_cu_count(int* n_cu) {
+  // a device's CU count never changes: asked of the runtime once per device, as every launch needs it
+  constexpr int kDevices = 64;
+  static std::atomic<int> known[kDevices];
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess && dev >= 0 && dev < kDevices) {
+    const int n = known[dev].load(std::memory_order_relaxed);
+    if (n > 0) {
+      *n_cu = n;
+      return dsa::ok();
+    }
+  }
   if (e == hipSuccess) e = hipDeviceGetAttribute(n_cu, hipDeviceAttributeMultiprocessorCount, dev);
   if (e != hipSuccess) return dsa::fail(DSA_ERR_LAUNCH, "dsa_device_cu_count: %s", hipGetErrorString(e));
+  if (dev >= 0 && dev < kDevices) known[dev].store(*n_cu, std::memory_order_relaxed);
   return dsa::ok();
 }

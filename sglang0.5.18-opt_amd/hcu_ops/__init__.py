@@ -146,10 +146,15 @@ def mqa_logits(q, kv_cache, weights, context_lens, block_table, max_context_len,
                 and hist_lens.shape[0] == rows and hist_lens.is_contiguous()
                 and _topk_splits(rows, max_context_len) > 1)
     fused = use_hist and rows <= hist_max_rows and rows_per_cta <= 3
-    logits, mask, zws = _C.mqa_logits_hist(q, kv_cache, weights, context_lens.view(-1), block_table,
-                                           max_context_len, group_size, persistent_ctas, rows_per_cta,
-                                           hist_lens if use_hist else None, fused)
-    _MQA_HIST = (logits, hist_lens, zws, fused) if use_hist else None
+    if context_lens.dim() != 1:
+        context_lens = context_lens.view(-1)
+    if not use_hist:
+        _MQA_HIST = None
+        return tuple(_C.mqa_logits(q, kv_cache, weights, context_lens, block_table, max_context_len, group_size,
+                                   persistent_ctas, rows_per_cta))
+    logits, mask, zws = _C.mqa_logits_hist(q, kv_cache, weights, context_lens, block_table, max_context_len,
+                                           group_size, persistent_ctas, rows_per_cta, hist_lens, fused)
+    _MQA_HIST = (logits, hist_lens, zws, fused)
     return logits, mask
 
 
