@@ -497,6 +497,18 @@ __device__ __forceinline__ uint32_t cand_digit(uint32_t key, const SampleCut& c)
   return d < 4095u ? d : 4095u;
 }
 
+// A K* of +0, the key of a masked-out token, means that zeros fill the row, and collecting
+// them would overflow any list.  It moves up to the positive keys: 2048 of them or more are resolved
+// as ever, fewer leave zeros to fill up with (sparse_row).  Before, the overflowing lists sent such rows
+// to the exact path (us a launch, 1500 positives a row: 64 x 65,536 71.0 -> 23.7, 1024 x 65,536 231 -> 87,
+// 32 x 16,384 32.0 -> 17.8; all zeros, 8 x 65,536 41.2 -> 20.5).  The long list's kernels, at 128 VGPRs,
+// have no room for it: their rows still take the exact path.
+constexpr uint32_t kPositive = kZeroKey + 1u;  // the smallest positive key; no other K* has it (a digit's edge)
+
+__device__ __forceinline__ void positives_only(SampleCut& c) {
+  if (c.thr == kZeroKey) c.thr = kPositive;
+}
+
 // Scratch of the threshold search (LDS).
 struct SampleLds {
   int* hist;      // kBins
@@ -1007,6 +1019,84 @@ __device__ __forceinline__ void exact_row(ResolveLds<NT, CAP>& L, const RowSrc& 
 __device__ __forceinline__ int sparse_fast_case(int n_pos, const SampleCut& cut) {
   if (n_pos != kTopK) return 0;
   return cut.thr <= kZeroKey + 1u ? 1 : -1;
+}
+
+// The first `need` tokens of key +0 in token order, as page-table entries from dst[kTopK - need] on;
+// false, with nothing usable written, when the row holds fewer.  A thread owns 16 consecutive tokens of
+// each 16 NT-token step; rows that come here are mostly zeros, so one step is the rule.
+template <bool kVec, int NT>
+__device__ __forceinline__ bool emit_zeros(const RowSrc& r, int need, const PtRow& pt, int32_t* dst, int* s_scan) {
+  constexpr int kStep = NT * 16;
+  const int base = kTopK - need;
+  int n = 0, parity = 0;
+  for (int b = 0; b < r.len && n < need; b += kStep) {  // block-uniform
+    const int i0 = b + static_cast<int>(threadIdx.x) * 16;
+    uint32_t f = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      uint32_t k[4];
+      const uint32_t v = load_keys4<kVec>(r, i0 + 4 * u, k);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f |= static_cast<uint32_t>(((v >> j) & 1u) && k[j] == kZeroKey) << (4 * u + j);
+    }
+    int total;
+    int p = n + block_prefix<NT, true>(__popc(f), total, s_scan, parity);
+    parity ^= 1;
+    for (; f && p < need; f &= f - 1, ++p) put(dst, base + p, i0 + static_cast<int>(__builtin_ctz(f)));
+    n += total;
+  }
+  if (n < need) return false;
+  __syncthreads();  // the token indices are there for every lane: turned into entries in one pass
+  constexpr int kPer = kTopK / NT;
+  int32_t tk[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = static_cast<int>(threadIdx.x) + j * NT;
+    tk[j] = i >= base ? dst[i] : 0;
+  }
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = static_cast<int>(threadIdx.x) + j * NT;
+    const int32_t e = pt.at(tk[j], true);
+    if (i >= base) dst[i] = e;
+  }
+  return true;
+}
+
+// A row whose n < 2048 positive keys are all collected (load as resolve_cands): the reference's sparse
+// fast path, threshold +0 -- the positives in token order, then the first zeros.  False when the row has
+// too few zeros for that (the 2048th key is negative): the caller runs exact_row.
+template <bool kVec, int NT, int CAP, typename Load>
+__device__ __forceinline__ bool sparse_row(ResolveLds<NT, CAP>& L, int n, const RowSrc& r, const PtRow& pt, int32_t* dst,
+                                           Load load) {
+  constexpr int EPT = kTopK / NT;
+  const int tid = threadIdx.x;
+  int tt[EPT];
+  int32_t pv[EPT];
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) {
+    const int e = tid + j * NT;
+    tt[j] = e < n ? load(e) : 0;
+  }
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) pv[j] = pt.at(tt[j], tid + j * NT < n);
+  uint32_t* bits = reinterpret_cast<uint32_t*>(L.hist);
+  constexpr int WPT = kBins / NT;
+  uint4* b4 = reinterpret_cast<uint4*>(bits + tid * WPT);
+#pragma unroll
+  for (int j = 0; j < WPT / 4; ++j) b4[j] = make_uint4(0u, 0u, 0u, 0u);
+  if (tid == 0) L.misc[3] = 0;
+  // (its barriers order the zeroed bitmap and the list's reads before the emission)
+  if (!emit_zeros<kVec, NT>(r, kTopK - n, pt, dst, L.scan)) return false;  // block-uniform
+  __syncthreads();
+  emit_held<NT>(
+      [&](auto&& fn) {
+#pragma unroll
+        for (int j = 0; j < EPT; ++j)
+          if (tid + j * NT < n) fn(tt[j], false, pv[j]);
+      },
+      &L.misc[3], bits, reinterpret_cast<uint16_t*>(L.ci + CAP - kBins / 2), L.wtot, r.len, dst);
+  return true;
 }
 
 // Resolves n (kTopK <= n <= CAP) collected candidates (keys >= cut.thr) that hold the row's top
@@ -1683,6 +1773,7 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
     // the last (a 4096-row prefill slab 327 -> 323 us; the decode split kernel unchanged).
     SampleCut cut = sample_threshold<kTs>(r, smp, S, [&]() { load_batch<kVec, kTs>(r, b0, x0); });
     load_batch<kVec, kTs>(r, b0 + kStep, x1);
+    if constexpr (CAP == kCapS) positives_only(cut);
     if (threadIdx.x == 0) L.misc[2] = 0;
     __syncthreads();
     collect_ge<kVec, kTs>(r, b0, (len + kStep - 1) / kStep, cut.thr, L.ck, L.ci, &L.misc[2], CAP, x0, x1);
@@ -1717,7 +1808,9 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
       __syncthreads();
       n = L.misc[2];
     }
-    if (n >= kTopK && n <= CAP) {  // block-uniform
+    if (CAP == kCapS && cut.thr == kPositive && n < kTopK) {  // block-uniform
+      if constexpr (CAP == kCapS) done = sparse_row<kVec>(L, n, r, pt, dst, [&](int e) { return L.ci[e] & 0x7FFFFFFF; });
+    } else if (n >= kTopK && n <= CAP) {  // block-uniform
       done = resolve_cands<kVec>(L, n, cut, r, pt, dst, [&](int e, uint32_t& k, int& t) {
         collected(L.ck[e], L.ci[e], k, t);
       });
@@ -1887,7 +1980,8 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
     Batch x0, x1;
     if (tid == 0) L.n[0] = 0;
     const SampleLds S{L.u.res.hist, L.wtot, L.res};
-    const SampleCut cut = sample_threshold<kTs>(r, smp, S, [&]() { load_batch<kVec, kTs>(rr, b0, x0); });
+    SampleCut cut = sample_threshold<kTs>(r, smp, S, [&]() { load_batch<kVec, kTs>(rr, b0, x0); });
+    if constexpr (CAP == kCapS) positives_only(cut);
     load_batch<kVec, kTs>(rr, b0 + kStep, x1);  // the second batch once K* is known (see the row kernel)
     collect_ge<kVec, kTs>(rr, b0, (end - begin + kStep - 1) / kStep, cut.thr, L.u.col.ck, L.u.col.ci, &L.n[0], CAP,
                           x0, x1);
@@ -1948,7 +2042,11 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
     if (!L.n[2]) return;
 
     const int n_tot = L.n[3];
-    if (n_tot >= kTopK && n_tot <= CAP) {  // block-uniform
+    if (CAP == kCapS && cut.thr == kPositive && n_tot < kTopK) {  // block-uniform
+      if constexpr (CAP == kCapS) done = sparse_row<kVec>(L.u.res, n_tot, r, pt_row(a, row), dst(), [&](int e) {
+        return __hip_atomic_load(&lt[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      });
+    } else if (n_tot >= kTopK && n_tot <= CAP) {  // block-uniform
       done = resolve_cands<kVec, true>(L.u.res, n_tot, cut, r, pt_row(a, row), dst(),
                                               [&](int e, uint32_t& k, int& t, int32_t& v) {
         k = __hip_atomic_load(&lk[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
