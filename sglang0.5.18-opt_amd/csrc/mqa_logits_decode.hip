@@ -675,8 +675,14 @@ int auto_rows(int heads, int group, int64_t batch, int64_t bt_pages, int64_t n_c
 // heads): 504 x 20,984, 32: 112 -> 54 (64 heads 158 -> 85); 1024 x 8192, 64: 125 -> 63; 904 x 5003, 64:
 // 79 -> 39; 64 x 60,064, 64: 227 -> 38; 16 x 30,016, 64: 224 -> 8.6; 2048 x 32,048, 32: 266 -> 242; a
 // 4096-row slab over 69,632 keys is the same for every L (1812-1822).  Over a sweep of L at each
-// shape the rule's time is within 7% of the best.
+// shape the rule's time is within 7% of the best.  From 2048 pages a CU on, where L makes no difference to
+// the time, the longest slices spare the re-reading of q, once a slice (a 4096-row slab over 73,728 keys
+// fetched 0.62 GB a launch with short slices, 0.28 GB with these).
 int64_t slice_pages_for(int64_t n_groups, int64_t width_pages, int64_t n_cu, int64_t max_pages) {
+  if (n_groups * width_pages >= 2048 * n_cu) {
+    const int64_t n = (width_pages + max_pages - 1) / max_pages;
+    return (width_pages + n - 1) / n;
+  }
   int64_t best = 1, best_cost = INT64_MAX;
   for (int64_t L = 1; L <= std::min(max_pages, width_pages); ++L) {
     const int64_t rounds = (n_groups * ((width_pages + L - 1) / L) + n_cu - 1) / n_cu;
