@@ -27,9 +27,9 @@
 //    chosen per (R, histogram) for LDS / register fit (Shape).
 //  * Balanced static grid: a row group is R rows of one request.  Every CTA reads the groups'
 //    lengths and gives group g ceil(pages_g * T / P) CTAs (P = total pages, T = the target CTA
-//    count), so each CTA streams ~P / T consecutive pages of a single group whatever the length
-//    mix; the grid (T + groups) depends only on shapes, so the launch can be captured in a
-//    hipGraph, and T is chosen so that every CTA is resident at once.
+//    count), but no more than one a page, so each CTA streams ~P / T consecutive pages of a single
+//    group whatever the length mix; the grid (T + groups) depends only on shapes, so the launch can be
+//    captured in a hipGraph, and T is chosen so that every CTA is resident at once.
 //  * Mask words past a group's pages are zeroed by the group's own CTAs (a share each, 8-B
 //    stores), so no separate mask memset is launched; a group with no pages still gets a CTA.
 //  * Prefill is the same kernel with a request's query rows as one group in CTAs of 8 rows:
@@ -113,7 +113,6 @@ struct DecodeArgs {
   int16_t* mask;
   int64_t mask_stride;
   int group;
-  int R;
   int n_groups;  // batch / R
   int target;    // T: CTAs the pages are spread over
   const int32_t* hist_lens;
@@ -135,21 +134,34 @@ __device__ __forceinline__ int scored_len(const DecodeArgs& a, int row) {
 }
 
 // Pages of row group g: ceil(max over its R rows of len / 64).
+template <int R>
 __device__ __forceinline__ int group_pages(const DecodeArgs& a, int g) {
+  int l[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) l[r] = a.ctx[g * R + r];
   int m = 0;
-  for (int r = 0; r < a.R; ++r) m = max(m, clamp_len(a.ctx[g * a.R + r], a.width));
+#pragma unroll
+  for (int r = 0; r < R; ++r) m = max(m, clamp_len(l[r], a.width));
   return (m + kPage - 1) / kPage;
 }
 
-// A group with no pages still gets one CTA: it zeroes the group's mask rows.
+// CTAs of a group: its share of the target, and no more than it has pages, but up to kZeroCtas to zero
+// the group's mask rows (one if it has no pages).  T comes from the block tables' width, so short requests
+// in wide tables have far fewer pages than T.  Capped, the CTAs with pages are the launch's first and lie
+// evenly over the XCDs and CUs; the others leave at once.  Spread over the whole share instead, every
+// CTA read the query fragments, and a power-of-two spacing put all the pages on the CTAs of one XCD (us a
+// launch, 32 heads, 131,072-token tables, requests x 6 rows: 1 of 2048 / 8192 / 32,768 tokens 7.3 / 8.1 /
+// 8.3 -> 5.0 / 4.9 / 6.1, 4 of 2048 / 8192 7.1 / 7.8 -> 5.2 / 6.2; 64 heads, 1 x 8 rows of 2048 8.8 -> 6.6).
+constexpr int kZeroCtas = 16;
 __device__ __forceinline__ int group_ctas(int pages, int total_pages, int target) {
   if (pages == 0) return 1;
-  return static_cast<int>((static_cast<int64_t>(pages) * target + total_pages - 1) / total_pages);
+  return min(static_cast<int>((static_cast<int64_t>(pages) * target + total_pages - 1) / total_pages),
+             max(pages, kZeroCtas));
 }
 
 // Work assignment, identical in every CTA: s_assign = {group (-1: none), index among the group's
 // CTAs, their count}; group g gets ceil(pages_g * T / P) CTAs.  Ends before a barrier (the caller's).
-template <int NT>
+template <int R, int NT>
 __device__ void assign_cta(const DecodeArgs& a, int (&s_w)[2][NT / kWave], int* s_assign) {
   const int tid = threadIdx.x;
   const int cta = blockIdx.x;
@@ -165,11 +177,11 @@ __device__ void assign_cta(const DecodeArgs& a, int (&s_w)[2][NT / kWave], int* 
   if (cached) {
 #pragma unroll
     for (int i = 0; i < kGpt; ++i) {
-      gp[i] = g_lo + i < g_hi ? group_pages(a, g_lo + i) : 0;
+      gp[i] = g_lo + i < g_hi ? group_pages<R>(a, g_lo + i) : 0;
       my_pages += gp[i];
     }
   } else {
-    for (int g = g_lo; g < g_hi; ++g) my_pages += group_pages(a, g);
+    for (int g = g_lo; g < g_hi; ++g) my_pages += group_pages<R>(a, g);
   }
   int total_pages;
   block_excl_sum<NT>(my_pages, total_pages, s_w[0]);
@@ -179,7 +191,7 @@ __device__ void assign_cta(const DecodeArgs& a, int (&s_w)[2][NT / kWave], int* 
 #pragma unroll
     for (int i = 0; i < kGpt; ++i) my_ctas += g_lo + i < g_hi ? group_ctas(gp[i], total_pages, a.target) : 0;
   } else {
-    for (int g = g_lo; g < g_hi; ++g) my_ctas += group_ctas(group_pages(a, g), total_pages, a.target);
+    for (int g = g_lo; g < g_hi; ++g) my_ctas += group_ctas(group_pages<R>(a, g), total_pages, a.target);
   }
   int total_ctas;
   int c0 = block_excl_sum<NT>(my_ctas, total_ctas, s_w[1]);
@@ -191,7 +203,7 @@ __device__ void assign_cta(const DecodeArgs& a, int (&s_w)[2][NT / kWave], int* 
 #pragma unroll
         for (int j = 1; j < kGpt; ++j) p = i == j ? gp[j] : p;
       } else {
-        p = group_pages(a, g_lo + i);
+        p = group_pages<R>(a, g_lo + i);
       }
       const int n = group_ctas(p, total_pages, a.target);
       if (cta < c0 + n) {
@@ -211,17 +223,18 @@ __device__ void assign_cta(const DecodeArgs& a, int (&s_w)[2][NT / kWave], int* 
 // different row groups: each XCD's L2 then holds one slice that all of its CTAs read, where the
 // group-major balanced grid has every XCD's resident CTAs spread over the whole K range (a prefill's
 // 10-20 MB of K misses the L2s).  A pair past its group's pages leaves at once.  The host sizes the
-// slices (slice_count); the lengths are read for the CTA's own group only (ranking the non-empty
+// slices (slice_pages_for); the lengths are read for the CTA's own group only (ranking the non-empty
 // pairs first read every group's twice, behind three barriers, and packed a causal launch no better).
 
 // The balanced assignment for up to 64 groups, computed by every wave on its own (lane g holds group g): no
 // LDS and no barrier before the CTA's first block-table read.  Returns {group (-1: none), index
 // within the group's CTAs, their count}, wave-uniform.
+template <int R>
 __device__ __forceinline__ int3 assign_cta_wave(const DecodeArgs& a) {
   const int lane = threadIdx.x & 63;
   const int cta = blockIdx.x;
   const bool in = lane < a.n_groups;
-  const int pages = in ? group_pages(a, lane) : 0;
+  const int pages = in ? group_pages<R>(a, lane) : 0;
   const int incl_p = wave_prefix_sum(pages);
   const int total = __builtin_amdgcn_readlane(incl_p, 63);
   const int ctas = in ? group_ctas(pages, total, a.target) : 0;
@@ -309,12 +322,12 @@ __global__ __launch_bounds__((Shape<H, R, kHist>::kThreads)) __attribute__((amdg
     grp = cta - jc * a.n_groups;
     nj = 1;
   } else if (a.n_groups <= kWave) {  // block-uniform
-    const int3 as = assign_cta_wave(a);
+    const int3 as = assign_cta_wave<R>(a);
     grp = uniform(as.x);
     jc = uniform(as.y);
     nj = uniform(as.z);
   } else {
-    assign_cta<NT>(a, s_w, s_assign);
+    assign_cta<R, NT>(a, s_w, s_assign);
     __syncthreads();
     grp = s_assign[0];
     jc = s_assign[1];
@@ -361,11 +374,42 @@ __global__ __launch_bounds__((Shape<H, R, kHist>::kThreads)) __attribute__((amdg
     p_begin = jc * a.slice_pages;
     p_end = min(p_begin + a.slice_pages, pages);
     if (p_begin >= p_end) return;  // no page of this group in the slice
+  } else if (pages < nj) {  // block-uniform: a page each for the group's first CTAs
+    p_begin = min(jc, pages);
+    p_end = min(jc + 1, pages);
   } else {
     p_begin = static_cast<int>(static_cast<int64_t>(pages) * jc / nj);
     p_end = static_cast<int>(static_cast<int64_t>(pages) * (jc + 1) / nj);
   }
   const int n_local = p_end - p_begin;  // <= Sh::kMaxPages by the host's choice of target
+  // Mask words of the group's rows past its pages (no CTA scores them) are zeroed by the
+  // group's CTAs, a share each: one 8-B store per page and row when the layout allows it.
+  // Issued after the page stream, so that no DMA wait covers these stores.
+  auto zero_mask_tail = [&]() {
+    const int tail = a.bt_pages - pages;
+    const int units = R * tail;
+    const int u0 = static_cast<int>(static_cast<int64_t>(units) * jc / nj);
+    const int u1 = static_cast<int>(static_cast<int64_t>(units) * (jc + 1) / nj);
+    const bool wide = (reinterpret_cast<uintptr_t>(a.mask) & 7u) == 0 && (a.mask_stride & 3) == 0;
+    for (int u = kMask && a.mask != nullptr ? u0 + tid : u1; u < u1; u += NT) {
+      const int rr = u / tail;
+      int16_t* m = a.mask + static_cast<int64_t>(row0 + rr) * a.mask_stride + (pages + u - rr * tail) * 4;
+      if (wide) {
+        *reinterpret_cast<uint64_t*>(m) = 0;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m[e] = 0;
+      }
+    }
+  };
+  // A CTA without a page (kZeroCtas) only zeroes its share.
+  if constexpr (!kHist) {
+    if (n_local == 0) {  // block-uniform
+      zero_mask_tail();
+      zero_share();
+      return;
+    }
+  }
   // the pages this wave scores: without a mask to write, those that hold tokens of its row
   const int n_mine = kMask ? n_local : min(n_local, (len + kPage - 1) / kPage - p_begin);
   const int32_t* btr = a.bt + static_cast<int64_t>(group_row) * a.bt_stride + p_begin;
@@ -407,27 +451,6 @@ __global__ __launch_bounds__((Shape<H, R, kHist>::kThreads)) __attribute__((amdg
     for (int i = tid; i < R * kBins / 2; i += NT) s_hist[i] = 0;
     if (tid < 2 * R) s_cnt[tid] = 0;
   }
-  // Mask words of the group's rows past its pages (no CTA scores them) are zeroed by the
-  // group's CTAs, a share each: one 8-B store per page and row when the layout allows it.
-  // Issued after the page stream, so that no DMA wait covers these stores.
-  auto zero_mask_tail = [&]() {
-    const int tail = a.bt_pages - pages;
-    const int units = R * tail;
-    const int u0 = static_cast<int>(static_cast<int64_t>(units) * jc / nj);
-    const int u1 = static_cast<int>(static_cast<int64_t>(units) * (jc + 1) / nj);
-    const bool wide = (reinterpret_cast<uintptr_t>(a.mask) & 7u) == 0 && (a.mask_stride & 3) == 0;
-    for (int u = kMask && a.mask != nullptr ? u0 + tid : u1; u < u1; u += NT) {
-      const int rr = u / tail;
-      int16_t* m = a.mask + static_cast<int64_t>(row0 + rr) * a.mask_stride + (pages + u - rr * tail) * 4;
-      if (wide) {
-        *reinterpret_cast<uint64_t*>(m) = 0;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m[e] = 0;
-      }
-    }
-  };
-
   int nz = 0, pos = 0;
   const int n_steps = (n_local + S - 1) / S;  // block-uniform
   const int t_lo = lane & 15;
@@ -655,7 +678,11 @@ void shape_host(int R, int& ctas_per_cu, int& max_pages) {
 // 46.5; 8 x 6, 16K-131K 37.5 -> 35.0 with three rows (35.7 with six: there the matrix work bounds both,
 // and a three-row CTA's shorter barriers win).  With few pages the launch is one latency chain and more,
 // smaller CTAs win (1 x 6 rows of 16,384 tokens, 256 pages: 5.1 with two rows, 5.7 with six; 2 x 4 of 4000:
-// 4.3 / 4.7; 4 x 4 of 30,000, 1876 pages: 12.8 / 11.5): four pages a CU is the line.
+// 4.3 / 4.7).  The line is four pages a CU of the tables' capacity, the contexts being on the device.  At
+// 1024 pages held the larger sets win (32 heads, 1 x 65,536 tokens: 4 rows 7.6 -> 6.9, 6 rows 8.9 -> 8.1, 8
+// rows 10.1 -> 8.8; 64 heads 9.8 -> 9.0, 10.8 -> 10.3, 11.9 -> 10.7).  Below it in a wide table (131,072
+// tokens) they win or tie from 256 pages held (1 x 16,384: 4.9 -> 4.7, 5.2 -> 5.0, 5.6 -> 5.4; 64 heads 5.4 ->
+// 5.4, 6.2 -> 5.9, 6.8 -> 6.7) and lose at 32 (1 x 2048: 4.4 -> 4.6, 5.0, 5.4; 64 heads 4.8 -> 5.2, 5.0, 6.6).
 int auto_rows(int heads, int group, int64_t batch, int64_t bt_pages, int64_t n_cu) {
   const int few = group % 2 == 0 ? 2 : 1;
   if (batch / group * bt_pages < 4 * n_cu) return few;
@@ -729,7 +756,6 @@ int enqueue(DecodeArgs a, int heads, int R, int target_ctas, bool hist, const in
   if (target * max_cta_pages < max_pages) target = (max_pages + max_cta_pages - 1) / max_cta_pages;
   const int64_t grid = target + n_groups;
   DSA_REQUIRE(grid <= 0x7FFFFFFF, "%s: grid too large", who);
-  a.R = R;
   a.n_groups = static_cast<int>(n_groups);
   // A logits block beyond half the chip's 32 MB of L2 streams out with nontemporal stores: the
   // block does not stay cached for the top-k anyway, and the launch then ends without a large
@@ -768,7 +794,6 @@ int enqueue_slices(DecodeArgs a, int heads, hipStream_t stream, const char* who)
   a.slice_pages = static_cast<int>(slice_pages_for(n_groups, width_pages, n_cu, max_cta_pages));
   const int64_t grid = n_groups * ((width_pages + a.slice_pages - 1) / a.slice_pages);
   DSA_REQUIRE(grid <= 0x7FFFFFFF, "%s: grid too large", who);
-  a.R = R;
   a.n_groups = static_cast<int>(n_groups);
   a.nt_logits = a.batch * static_cast<int64_t>(a.width) * 4 > (16ll << 20) ? 1 : 0;
   const uint32_t g = static_cast<uint32_t>(grid);
