@@ -676,7 +676,9 @@ void shape_host(int R, int& ctas_per_cu, int& max_pages) {
 // requests x rows, tokens): 32 heads 8 x 6, 73,000 40.5 -> 24.7; 32 x 6, 8K-30K 39.7 -> 24.6; 64 x 4, 2K-50K
 // 67.9 -> 57.9; 16 x 8, 20K-60K 45.2 -> 30.2; 64 heads 64 x 4, 2K-50K 79.7 -> 68.5; 16 x 8, 20K-60K 53.9 ->
 // 46.5; 8 x 6, 16K-131K 37.5 -> 35.0 with three rows (35.7 with six: there the matrix work bounds both,
-// and a three-row CTA's shorter barriers win).  With few pages the launch is one latency chain and more,
+// and a three-row CTA's shorter barriers win).  Larger groups at 64 heads: three rows are no better than two
+// (32 x 12, 32,768 141 -> 147; 16 x 18, 32,768 101 -> 104), four are (32 x 12, 32,768 141 -> 131; 4 x 12,
+// 131,072 76 -> 67; 32 x 12, 8192 43.6 -> 38.3).  With few pages the launch is one latency chain and more,
 // smaller CTAs win (1 x 6 rows of 16,384 tokens, 256 pages: 5.1 with two rows, 5.7 with six; 2 x 4 of 4000:
 // 4.3 / 4.7).  The line is four pages a CU of the tables' capacity, the contexts being on the device.  At
 // 1024 pages held the larger sets win (32 heads, 1 x 65,536 tokens: 4 rows 7.6 -> 6.9, 6 rows 8.9 -> 8.1, 8
@@ -687,9 +689,9 @@ int auto_rows(int heads, int group, int64_t batch, int64_t bt_pages, int64_t n_c
   const int few = group % 2 == 0 ? 2 : 1;
   if (batch / group * bt_pages < 4 * n_cu) return few;
   if (group % 8 == 0) return 8;
-  if (group % 6 == 0) return heads == 32 ? 6 : 3;
+  if (group % 6 == 0 && heads == 32) return 6;
   if (group % 4 == 0) return 4;
-  return few;
+  return group == 6 ? 3 : few;
 }
 
 // Pages of the slices a prefill launch of n_groups 8-row groups cuts its width_pages K pages into

@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("heads", [32, 64])
-@pytest.mark.parametrize("group,bt_pages", [(2, 700), (4, 40), (4, 700), (6, 700), (8, 600), (10, 700), (12, 700)])
+@pytest.mark.parametrize("group,bt_pages", [(2, 700), (4, 40), (4, 700), (6, 700), (8, 600), (10, 700), (12, 700),
+                                             (18, 700)])
 def test_open_rows_per_cta(gpu, heads, group, bt_pages):
     case = wl.decode_case(40 + group, [2100, 0, 63, 1], group=group, heads=heads, bt_pages=bt_pages)
     q8, w = hcu_ops.quant_q_fp8(case.q.to(gpu), case.w.to(gpu))
