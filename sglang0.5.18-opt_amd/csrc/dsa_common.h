@@ -170,10 +170,9 @@ __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirs
 // barrier; s_w (NT / 64 words) must not be reused before the next barrier.
 template <int NT>
 __device__ __forceinline__ int block_excl_sum(int x, int& total, int* s_w) {
-  const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int inc = wave_prefix_sum(x);
-  if (lane == 63) s_w[w] = inc;
+  if (lane_id() == kWave - 1) s_w[w] = inc;
   __syncthreads();
   int before = 0, tot = 0;
 #pragma unroll

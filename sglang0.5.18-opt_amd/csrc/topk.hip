@@ -501,8 +501,8 @@ __device__ __forceinline__ uint32_t cand_digit(uint32_t key, const SampleCut& c)
 // them would overflow any list.  It moves up to the positive keys: 2048 of them or more are resolved
 // as ever, fewer leave zeros to fill up with (sparse_row).  Before, the overflowing lists sent such rows
 // to the exact path (us a launch, 1500 positives a row: 64 x 65,536 71.0 -> 23.7, 1024 x 65,536 231 -> 87,
-// 32 x 16,384 32.0 -> 17.8; all zeros, 8 x 65,536 41.2 -> 20.5).  The long list's kernels, at 128 VGPRs,
-// have no room for it: their rows still take the exact path.
+// 32 x 16,384 32.0 -> 17.8; all zeros, 8 x 65,536 41.2 -> 20.5).  The long list's kernels and the one-CTA
+// kernel for unaligned rows, at 128 VGPRs, have no room for it: their rows still take the exact path.
 constexpr uint32_t kPositive = kZeroKey + 1u;  // the smallest positive key; no other K* has it (a digit's edge)
 
 __device__ __forceinline__ void positives_only(SampleCut& c) {
@@ -1748,6 +1748,7 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
   } lds;
   ResolveLds<kTs, CAP>& L = lds.res;
   constexpr int kStep = kTs * 4 * kUnroll;
+  constexpr bool kFillZeros = kVec && CAP == kCapS;  // (the others have no registers left for it)
   const int row = blockIdx.x;
   const int len = row_len(a, row);
   const PtRow pt = pt_row(a, row);
@@ -1773,7 +1774,7 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
     // the last (a 4096-row prefill slab 327 -> 323 us; the decode split kernel unchanged).
     SampleCut cut = sample_threshold<kTs>(r, smp, S, [&]() { load_batch<kVec, kTs>(r, b0, x0); });
     load_batch<kVec, kTs>(r, b0 + kStep, x1);
-    if constexpr (CAP == kCapS) positives_only(cut);
+    if constexpr (kFillZeros) positives_only(cut);
     if (threadIdx.x == 0) L.misc[2] = 0;
     __syncthreads();
     collect_ge<kVec, kTs>(r, b0, (len + kStep - 1) / kStep, cut.thr, L.ck, L.ci, &L.misc[2], CAP, x0, x1);
@@ -1808,8 +1809,8 @@ __global__ __launch_bounds__(kTs) __attribute__((amdgpu_waves_per_eu(4))) void t
       __syncthreads();
       n = L.misc[2];
     }
-    if (CAP == kCapS && cut.thr == kPositive && n < kTopK) {  // block-uniform
-      if constexpr (CAP == kCapS) done = sparse_row<kVec>(L, n, r, pt, dst, [&](int e) { return L.ci[e] & 0x7FFFFFFF; });
+    if (kFillZeros && cut.thr == kPositive && n < kTopK) {  // block-uniform
+      if constexpr (kFillZeros) done = sparse_row<kVec>(L, n, r, pt, dst, [&](int e) { return L.ci[e] & 0x7FFFFFFF; });
     } else if (n >= kTopK && n <= CAP) {  // block-uniform
       done = resolve_cands<kVec>(L, n, cut, r, pt, dst, [&](int e, uint32_t& k, int& t) {
         collected(L.ck[e], L.ci[e], k, t);
@@ -2311,8 +2312,8 @@ int topk_common(const float* score, int64_t score_stride, int64_t width, int64_t
         else launch_held<256, 4>(a, vec, stream);
       } else if (vec && wide) hipLaunchKernelGGL((topk_row_sampled_kernel<true, kCapW>), grid_rows, dim3(kTs), 0, stream, a);
       else if (vec) hipLaunchKernelGGL((topk_row_sampled_kernel<true, kCapS>), grid_rows, dim3(kTs), 0, stream, a);
-      // unaligned rows always take the long list: its late page-table gather leaves room for the buffer loads
-      else hipLaunchKernelGGL((topk_row_sampled_kernel<false, kCapW>), grid_rows, dim3(kTs), 0, stream, a);
+      else if (wide) hipLaunchKernelGGL((topk_row_sampled_kernel<false, kCapW>), grid_rows, dim3(kTs), 0, stream, a);
+      else hipLaunchKernelGGL((topk_row_sampled_kernel<false, kCapS>), grid_rows, dim3(kTs), 0, stream, a);
     }
     return check_launch(who);
   }
