@@ -81,3 +81,31 @@ def test_held_rows(gpu, kind, rows, width, pad):
         got = hcu_ops.sparse_mask_topk_transform(score, m.to(gpu), lens.to(gpu), pt.to(gpu), cu).cpu().numpy()
         bad = [r for r in range(rows) if not np.array_equal(got[r], want[r])]
         assert not bad, f"{kind}, masked: rows {bad[:5]} (lengths {[int(lens[r]) for r in bad[:5]]})"
+
+
+@pytest.mark.parametrize("rows,width", [(6, 4096), (6, 4090), (6, 8192), (300, 4096)])
+@pytest.mark.parametrize("neg", ["normal", "ties", "zeros", "minus_zero", "inf"])
+def test_held_rows_threshold_near_zero(gpu, rows, width, neg):
+    """2048 positive keys give or take a few up to an eighth of the row, so that the search starts from zero or
+    just does not; the others negative, tied, +0, -0 or -inf."""
+    g = torch.Generator().manual_seed(width + rows)
+    lens = torch.randint(3000, width + 1, (rows,), generator=g, dtype=torch.int32)
+    lens[0], lens[1] = width, 2100
+    x = -torch.rand(rows, width, generator=g)
+    if neg == "ties":
+        x = torch.full((rows, width), -0.25)
+    elif neg in ("zeros", "minus_zero"):
+        x = torch.where(torch.rand(rows, width, generator=g) < 0.05, x, 0.0 if neg == "zeros" else -0.0)
+    elif neg == "inf":
+        x = torch.where(torch.rand(rows, width, generator=g) < 0.5, x, -float("inf"))
+    for r in range(rows):
+        n = int(lens[r])
+        off = [0, 1, -1, 70, -70, n // 16, -(n // 16), n // 8, -(n // 8)][r % 9]
+        at = torch.randperm(n, generator=g)[:max(0, min(n, 2048 + off))]
+        x[r, at] = torch.rand(at.numel(), generator=g) * (1e-30 if r % 2 else 3.0) + 1e-38
+    pt = torch.randperm(width, generator=g).to(torch.int32).repeat(rows, 1).contiguous()
+    cu = torch.arange(rows + 1, dtype=torch.int32, device=gpu)
+    want = topk_radix(x.numpy(), None, lens.numpy(), pt.numpy(), width)
+    got = hcu_ops.topk_transform(x.to(gpu), lens.to(gpu), pt.to(gpu), cu, max_splits=1).cpu().numpy()
+    bad = [r for r in range(rows) if not np.array_equal(got[r], want[r])]
+    assert not bad, f"rows {bad[:5]} (lengths {[int(lens[r]) for r in bad[:5]]})"
