@@ -226,8 +226,8 @@ int dsa_topk_transform_blocks(const float* score, int64_t score_stride, int64_t 
  *   out[r, :] = the top-2048 (ties to the lower token) of row r's logits over keys t < lens[r],
  *               as page_table[t], -1 padded when min(lens[r], width) < 2048.
  * q8 / w / kv_cache / block_table / lens as in dsa_mqa_logits_prefill; out int32 [rows, 2048].
- * dsa_prefill_slab_rows gives the slab size a byte budget of logits allows (a multiple of 8
- * rows when at least 8 fit, capped at max_slab_rows > 0 and at rows);
+ * dsa_prefill_slab_rows gives the slab size a byte budget of logits (rows padded to 128 B) allows (a
+ * multiple of 8 rows when at least 8 fit, capped at max_slab_rows > 0 and at rows; never less than one row);
  * dsa_prefill_indexer_workspace_bytes the workspace (256-B aligned) for rows padded to 128 B; one
  * without room for the pad (the logits slab of `width` floats a row, up to 256 B, then the top-k's
  * workspace) is taken too and holds unpadded rows. */

@@ -19,15 +19,6 @@ namespace {
 
 constexpr int64_t kSlabAlign = 8;  // the logits kernel scores a request's rows in CTAs of 8
 
-int64_t slab_rows_of(int64_t rows, int64_t width, int64_t max_slab_rows, int64_t budget_bytes) {
-  const int64_t row_bytes = width * static_cast<int64_t>(sizeof(float));
-  int64_t s = budget_bytes > 0 ? budget_bytes / row_bytes : rows;
-  if (max_slab_rows > 0 && s > max_slab_rows) s = max_slab_rows;
-  if (s >= kSlabAlign) s -= s % kSlabAlign;
-  if (s > rows) s = rows;
-  return s < 1 ? 1 : s;
-}
-
 size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 // Row stride of a slab's logits: whole 128-B lines.  With the keys' own count as the stride, three
@@ -35,6 +26,15 @@ size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 // logits kernel's 256-B stores straddle lines (4093 rows x 69,629 keys, 64 heads: 2182 -> 2075 us; a prompt
 // of 5003 tokens 273 -> 262).
 int64_t slab_stride(int64_t width) { return (width + 31) / 32 * 32; }
+
+int64_t slab_rows_of(int64_t rows, int64_t width, int64_t max_slab_rows, int64_t budget_bytes) {
+  const int64_t row_bytes = slab_stride(width) * static_cast<int64_t>(sizeof(float));
+  int64_t s = budget_bytes > 0 ? budget_bytes / row_bytes : rows;
+  if (max_slab_rows > 0 && s > max_slab_rows) s = max_slab_rows;
+  if (s >= kSlabAlign) s -= s % kSlabAlign;
+  if (s > rows) s = rows;
+  return s < 1 ? 1 : s;
+}
 
 size_t workspace_bytes_of(int64_t rows, int64_t width, int64_t stride, int64_t slab, int max_splits, int n_cu) {
   // the top-k of a slab may split rows only when the slab is the whole (short) input

@@ -139,6 +139,24 @@ def test_prefill_slab_policy(lib):
     assert small > (4 * 70000 * 4 + 255) // 256 * 256  # four 70K rows split: the top-k's workspace too
 
 
+def test_prefill_slab_holds_its_budget(lib):
+    """The logits slab of the workspace (rows padded to 128 B) stays within the byte budget its rows were taken
+    from, at key counts that do not fill a line."""
+    I64, I = ctypes.c_int64, ctypes.c_int
+    lib.dsa_prefill_slab_rows.argtypes = [I64, I64, I64, I64]
+    lib.dsa_prefill_slab_rows.restype = I64
+    lib.dsa_prefill_indexer_workspace_bytes.argtypes = [I64, I64, I64, I, I]
+    lib.dsa_prefill_indexer_workspace_bytes.restype = ctypes.c_size_t
+    for width in (1, 31, 32, 33, 1039, 5003, 69629, 131073):
+        for rows in (9, 64, 4096):
+            budget = (rows * width * 4 + 255) // 256 * 256
+            slab = lib.dsa_prefill_slab_rows(1 << 20, width, 0, budget)
+            if slab > 1:
+                need = lib.dsa_prefill_indexer_workspace_bytes(1 << 20, width, slab, 1, 256)
+                assert need <= budget, f"{slab} rows of {width} keys: {need} bytes for a budget of {budget}"
+
+
+
 def test_reference_knob_gate(monkeypatch):
     """mqa_logits pairs with the top-k only where the reference's gate would: the split top-k
     must split rows (reference hcu_ops/hcu_ops/__init__.py:96-98).  MI355X: 256 CUs."""
