@@ -135,8 +135,8 @@ int dsa_mqa_logits_prefill(const uint8_t* q8, const float* w, int heads, int64_t
                            float* logits, int64_t logits_stride, int64_t width,
                            hipStream_t stream);
 /* K pages a CTA of a dsa_mqa_logits_prefill launch streams on a device of n_cu CUs (a diagnostic: the launch
- * does not need it); 0 for up to 4 rows, whose CTAs share the pages evenly. */
-int dsa_prefill_slice_pages(int64_t rows, int64_t width, int n_cu);
+ * does not need it); 0 for the 1, 2 or 4 rows whose CTAs share the pages evenly. */
+int dsa_prefill_slice_pages(int heads, int64_t rows, int64_t width, int n_cu);
 
 /* ---------------------------------------------------------------------------------------------
  * Exact top-2048 + page-table transform over (sparse-mask) indexer logits (replaces hcu_ops

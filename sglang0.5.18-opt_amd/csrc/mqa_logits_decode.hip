@@ -728,7 +728,16 @@ int64_t slice_pages_for(int64_t n_groups, int64_t width_pages, int64_t n_cu, int
   return best;
 }
 
-constexpr int64_t kDecodeGridRows = 4;  // prefill calls of up to this many rows take the decode grid
+// Whether a prefill call takes the decode grid, one launch in CTAs of all its rows: 1, 2 and 4 rows; any
+// other count one short 8-row group.  Measured, decode grid / 8-row group (us; 64 heads, keys 4096, 30,004,
+// 131,072): 1 row 4.5 / 5.5, 5.2 / 7.7, 8.4 / 10.1; 2 rows 4.6 / 5.5, 5.5 / 7.7, 9.9 / 10.7; 4 rows 5.2 /
+// 5.5, 6.5 / 7.8, 10.7 / 11.0; 32 heads 1 row 4.2 / 4.5, 4.7 / 5.6, 7.4 / 7.6; 2 rows 4.3 / 4.5, 4.8 / 5.7, 7.7
+// / 7.8; 4 rows 4.7 / 4.5, 5.4 / 5.8, 8.8 / 8.1 and at 65,536 7.0 / 6.6, hence its line at four pages a CU.
+// Three rows as launches of two and one: 8.1 / 5.5, 9.6 / 7.8, 17.3 / 10.8.
+bool decode_grid(int heads, int64_t rows, int64_t width, int64_t n_cu) {
+  if (rows == 4) return heads == 64 || (width + kPage - 1) / kPage < 4 * n_cu;
+  return rows == 1 || rows == 2;
+}
 
 // Enqueues the kernel for a.batch rows in groups of R (a.group rows share a block-table row;
 // a.width caps the lengths).  a's pointers, strides and sizes are set and checked by the caller.
@@ -791,14 +800,11 @@ int enqueue(DecodeArgs a, int heads, int R, int target_ctas, bool hist, const in
 
 // The same for a.batch rows of one request in groups of 8 (the last one may be short), no mask: the
 // (slice, group) pairs of slice_pages_for.
-int enqueue_slices(DecodeArgs a, int heads, hipStream_t stream, const char* who) {
+int enqueue_slices(DecodeArgs a, int heads, int n_cu, hipStream_t stream, const char* who) {
   constexpr int R = 8;
   const int64_t n_groups = (a.batch + R - 1) / R;
-  int n_cu = 0;
-  const int st = dsa_device_cu_count(&n_cu);
-  if (st != DSA_OK) return st;
   const int64_t width_pages = (a.width + kPage - 1) / kPage;
-  a.slice_pages = dsa_prefill_slice_pages(a.batch, a.width, n_cu);
+  a.slice_pages = static_cast<int>(slice_pages_for(n_groups, width_pages, n_cu, Shape<64, R, false>::kMaxPages));
   const int64_t grid = n_groups * ((width_pages + a.slice_pages - 1) / a.slice_pages);
   DSA_REQUIRE(grid <= 0x7FFFFFFF, "%s: grid too large", who);
   a.n_groups = static_cast<int>(n_groups);
@@ -880,8 +886,8 @@ extern "C" int dsa_mqa_logits_decode(const uint8_t* q8, const float* w, int head
 // once per 8 query rows), the last group short when the count is not a multiple of 8: launches of their
 // own for a remainder's 4, 2 and 1 rows read the whole of K again, one after the other (us, launches of
 // their own -> one short group, 64 heads: 7 x 3007 12.1 -> 5.3; 39 x 1039 16.6 -> 5.3; 15 x 100,015 37.1
-// -> 19.2; 5 x 30,005 10.3 -> 7.6; 509 x 20,989, 32 heads 62 -> 54).  Up to 4 rows take the decode grid
-// in groups of 4, 2 and 1 (4 x 30,004: 6.0).  No mask is written.
+// -> 19.2; 5 x 30,005 10.3 -> 7.6; 509 x 20,989, 32 heads 62 -> 54).  1, 2 and 4 rows take the decode
+// grid (decode_grid).  No mask is written.
 int dsa::mqa_logits_prefill_over(const uint8_t* q8, const float* w, int heads, int64_t rows, const uint8_t* kv_cache,
                                  int64_t page_stride_bytes, const int32_t* block_table, int64_t bt_pages,
                                  const int32_t* lens, float* logits, int64_t logits_stride, int64_t width,
@@ -897,38 +903,33 @@ int dsa::mqa_logits_prefill_over(const uint8_t* q8, const float* w, int heads, i
                   (reinterpret_cast<uintptr_t>(kv_cache) & 15u) == 0 && (reinterpret_cast<uintptr_t>(q8) & 15u) == 0,
               "dsa_mqa_logits_prefill: kv_cache pages (stride >= 8448, %% 16) and q8 must be 16-B aligned");
   if (width <= min_len) return ok();  // no row is longer
-  int64_t done = 0;
-  for (const int R : {8, 4, 2, 1}) {
-    const int64_t left = rows - done;
-    const int64_t n = R == 8 ? (left > kDecodeGridRows ? left : 0) : left / R * R;
-    if (n == 0) continue;
-    DecodeArgs a{};
-    a.q8 = q8 + done * heads * kHeadDim;
-    a.w = w + done * heads;
-    a.kv = kv_cache;
-    a.page_stride = page_stride_bytes;
-    a.ctx = lens + done;
-    a.bt = block_table;
-    a.bt_stride = bt_pages;
-    a.bt_pages = static_cast<int>(bt_pages);
-    a.width = static_cast<int>(width);
-    a.logits = logits + done * logits_stride;
-    a.logits_stride = logits_stride;
-    a.mask = nullptr;
-    a.mask_stride = 0;
-    a.group = static_cast<int>(n);
-    a.batch = n;
-    a.min_len = min_len;
-    const int st = R == 8 ? enqueue_slices(a, heads, stream, "dsa_mqa_logits_prefill")
-                          : enqueue(a, heads, R, 0, false, nullptr, nullptr, stream, "dsa_mqa_logits_prefill");
-    if (st != DSA_OK) return st;
-    done += n;
-  }
-  return ok();
+  int n_cu = 0;
+  const int st = dsa_device_cu_count(&n_cu);
+  if (st != DSA_OK) return st;
+  DecodeArgs a{};
+  a.q8 = q8;
+  a.w = w;
+  a.kv = kv_cache;
+  a.page_stride = page_stride_bytes;
+  a.ctx = lens;
+  a.bt = block_table;
+  a.bt_stride = bt_pages;
+  a.bt_pages = static_cast<int>(bt_pages);
+  a.width = static_cast<int>(width);
+  a.logits = logits;
+  a.logits_stride = logits_stride;
+  a.mask = nullptr;
+  a.mask_stride = 0;
+  a.group = static_cast<int>(rows);
+  a.batch = rows;
+  a.min_len = min_len;
+  if (decode_grid(heads, rows, width, n_cu))
+    return enqueue(a, heads, static_cast<int>(rows), 0, false, nullptr, nullptr, stream, "dsa_mqa_logits_prefill");
+  return enqueue_slices(a, heads, n_cu, stream, "dsa_mqa_logits_prefill");
 }
 
-extern "C" int dsa_prefill_slice_pages(int64_t rows, int64_t width, int n_cu) {
-  if (rows <= kDecodeGridRows || width <= 0 || n_cu <= 0) return 0;
+extern "C" int dsa_prefill_slice_pages(int heads, int64_t rows, int64_t width, int n_cu) {
+  if (rows <= 0 || width <= 0 || n_cu <= 0 || decode_grid(heads, rows, width, n_cu)) return 0;
   return static_cast<int>(slice_pages_for((rows + 7) / 8, (width + kPage - 1) / kPage, n_cu, Shape<64, 8, false>::kMaxPages));
 }
 

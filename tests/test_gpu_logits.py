@@ -172,9 +172,11 @@ def test_decode_topk_counters_zeroed(gpu, group, lens):
     _check_decode(case, lg, mask)
 
 
-# row counts cover every launch split of the prefill entry: groups of 8, then of 4 and 1-3 rows
+# row counts cover every launch of the prefill entry: the decode grid (1, 2 and 4 rows) and groups of 8, the last one full
+# or short
 @pytest.mark.parametrize("heads,n_q,prefix", [(64, 40, 3000), (32, 9, 130), (64, 17, 0), (64, 15, 700),
-                                              (32, 6, 4100), (64, 3, 64)])
+                                              (32, 6, 4100), (64, 3, 64), (32, 3, 9000), (64, 4, 5000), (32, 4, 300),
+                                              (32, 4, 66000), (32, 2, 700), (64, 1, 4095)])
 def test_prefill_logits(gpu, heads, n_q, prefix):
     case = wl.prefill_case(21 + n_q, n_q, prefix, heads=heads)
     q8, w = hcu_ops.quant_q_fp8(case.q.to(gpu), case.w.to(gpu))

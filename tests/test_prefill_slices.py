@@ -15,7 +15,7 @@ STAGE = 255  # pages of a CTA's block-table slice
 def slice_pages():
     lib = ctypes.CDLL(os.path.join(os.path.dirname(hcu_ops.__file__), "libdsa_indexer.so"))
     f = lib.dsa_prefill_slice_pages
-    f.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    f.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
     return f
 
 
@@ -36,10 +36,19 @@ def test_slices_are_the_cheapest(slice_pages):
     for cus in (64, 256):
         for groups in (1, 2, 7, 33, 64, 113, 256, 511, 512, 626, 2048):
             for pages in (1, 2, 17, 64, 79, 128, 255, 256, 328, 501, 939, 1023, 1024, 1152, 2304):
-                got = slice_pages(groups * 8, pages * 64, cus)
-                assert got == cheapest(groups, pages, cus), (groups, pages, cus)
-                assert 1 <= got <= STAGE
-    assert slice_pages(4, 4096, 256) == 0 and slice_pages(0, 4096, 256) == 0  # up to four rows: the decode grid
+                for heads in (32, 64):
+                    got = slice_pages(heads, groups * 8, pages * 64, cus)
+                    assert got == cheapest(groups, pages, cus), (groups, pages, cus)
+                    assert 1 <= got <= STAGE
+
+
+def test_few_rows_are_one_launch(slice_pages):
+    """1, 2 and 4 rows share the pages evenly (0); three rows are a short 8-row group, not launches of two and one
+    that read every key twice."""
+    for heads in (32, 64):
+        for width in (100, 30004, 65472):
+            assert [slice_pages(heads, rows, width, 256) > 0 for rows in range(0, 10)] == [False] * 3 + [True, False] + [True] * 5
+    assert slice_pages(32, 4, 65537, 256) > 0 and slice_pages(64, 4, 65537, 256) == 0
 
 
 def test_rule_costs_little_host_time(slice_pages):
@@ -48,7 +57,7 @@ def test_rule_costs_little_host_time(slice_pages):
         for _ in range(15):
             t = time.perf_counter()
             for _ in range(500):
-                slice_pages(rows, width, 256)
+                slice_pages(64, rows, width, 256)
             t = (time.perf_counter() - t) / 500 * 1e9
             best = t if best is None else min(best, t)
         return best
