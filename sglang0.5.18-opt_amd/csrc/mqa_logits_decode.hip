@@ -703,12 +703,14 @@ int auto_rows(int heads, int group, int64_t batch, int64_t bt_pages, int64_t n_c
 // block-table stage allows, which left the chip idle for a chunk of few rows (us a launch; rows x keys,
 // heads): 504 x 20,984, 32: 112 -> 54 (64 heads 158 -> 85); 1024 x 8192, 64: 125 -> 63; 904 x 5003, 64:
 // 79 -> 39; 64 x 60,064, 64: 227 -> 38; 16 x 30,016, 64: 224 -> 8.6; 2048 x 32,048, 32: 266 -> 242; a
-// 4096-row slab over 69,632 keys is the same for every L (1812-1822).  Over a sweep of L at each
-// shape the rule's time is within 7% of the best.  From 2048 pages a CU on, where L makes no difference to
-// the time, the longest slices spare the re-reading of q, once a slice (a 4096-row slab over 73,728 keys
-// fetched 0.62 GB a launch with short slices, 0.28 GB with these).
-int64_t slice_pages_for(int64_t n_groups, int64_t width_pages, int64_t n_cu, int64_t max_pages) {
-  if (n_groups * width_pages >= 2048 * n_cu) {
+// 4096-row slab over 69,632 keys is the same for every L (1812-1822).  Over a sweep of L at 23
+// shapes the rule's time is within 12% of the best (median 5%).  64-head launches of a group a CU and 2048 pages a CU take
+// the longest slices, which spare the re-reading of q, once a slice (a 4096-row slab over 73,728 keys fetched
+// 0.62 GB a launch with short slices, 0.28 GB with these): 4096 x 65,536 1789 -> 1767 us, x 81,920 2247 -> 2244,
+// 2048 x 131,072 1811 -> 1802.  Below either count they lose (1024 x 131,072 909 -> 944, x 262,144 1820 -> 1870), and
+// with 32 heads throughout (4096 x 65,536 1007 -> 1023, x 81,920 1232 -> 1266, 2048 x 131,072 1048 -> 1068).
+int64_t slice_pages_for(int heads, int64_t n_groups, int64_t width_pages, int64_t n_cu, int64_t max_pages) {
+  if (heads == 64 && n_groups >= n_cu && n_groups * width_pages >= 2048 * n_cu) {
     const int64_t n = (width_pages + max_pages - 1) / max_pages;
     return (width_pages + n - 1) / n;
   }
@@ -804,7 +806,7 @@ int enqueue_slices(DecodeArgs a, int heads, int n_cu, hipStream_t stream, const 
   constexpr int R = 8;
   const int64_t n_groups = (a.batch + R - 1) / R;
   const int64_t width_pages = (a.width + kPage - 1) / kPage;
-  a.slice_pages = static_cast<int>(slice_pages_for(n_groups, width_pages, n_cu, Shape<64, R, false>::kMaxPages));
+  a.slice_pages = static_cast<int>(slice_pages_for(heads, n_groups, width_pages, n_cu, Shape<64, R, false>::kMaxPages));
   const int64_t grid = n_groups * ((width_pages + a.slice_pages - 1) / a.slice_pages);
   DSA_REQUIRE(grid <= 0x7FFFFFFF, "%s: grid too large", who);
   a.n_groups = static_cast<int>(n_groups);
@@ -930,7 +932,8 @@ int dsa::mqa_logits_prefill_over(const uint8_t* q8, const float* w, int heads, i
 
 extern "C" int dsa_prefill_slice_pages(int heads, int64_t rows, int64_t width, int n_cu) {
   if (rows <= 0 || width <= 0 || n_cu <= 0 || decode_grid(heads, rows, width, n_cu)) return 0;
-  return static_cast<int>(slice_pages_for((rows + 7) / 8, (width + kPage - 1) / kPage, n_cu, Shape<64, 8, false>::kMaxPages));
+  return static_cast<int>(
+      slice_pages_for(heads, (rows + 7) / 8, (width + kPage - 1) / kPage, n_cu, Shape<64, 8, false>::kMaxPages));
 }
 
 extern "C" int dsa_mqa_logits_prefill(const uint8_t* q8, const float* w, int heads, int64_t rows,

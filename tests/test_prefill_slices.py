@@ -19,9 +19,10 @@ def slice_pages():
     return f
 
 
-def cheapest(groups, pages, cus):
-    """The first slice length of least cost (sixths of a page); the longest slices from 2048 pages a CU on."""
-    if groups * pages >= 2048 * cus:
+def cheapest(heads, groups, pages, cus):
+    """The first slice length of least cost (sixths of a page); for 64 heads the longest slices from a group and 2048
+    pages a CU on."""
+    if heads == 64 and groups >= cus and groups * pages >= 2048 * cus:
         n = -(-pages // STAGE)
         return -(-pages // n)
 
@@ -38,7 +39,7 @@ def test_slices_are_the_cheapest(slice_pages):
             for pages in (1, 2, 17, 64, 79, 128, 255, 256, 328, 501, 939, 1023, 1024, 1152, 2304):
                 for heads in (32, 64):
                     got = slice_pages(heads, groups * 8, pages * 64, cus)
-                    assert got == cheapest(groups, pages, cus), (groups, pages, cus)
+                    assert got == cheapest(heads, groups, pages, cus), (heads, groups, pages, cus)
                     assert 1 <= got <= STAGE
 
 
