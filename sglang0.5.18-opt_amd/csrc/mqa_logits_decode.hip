@@ -145,13 +145,15 @@ __device__ __forceinline__ int group_pages(const DecodeArgs& a, int g) {
   return (m + kPage - 1) / kPage;
 }
 
+// (The loops over a thread's groups below stay rolled: unrolled, their 64-bit divisions are a fifth of the kernel,
+// whose code every launch fetches again, 0.1 us.)
 // CTAs of a group: its share of the target, and no more than it has pages, but up to kZeroCtas to zero
 // the group's mask rows (one if it has no pages).  T comes from the block tables' width, so short requests
 // in wide tables have far fewer pages than T.  Capped, the CTAs with pages are the launch's first and lie
 // evenly over the XCDs and CUs; the others leave at once.  Spread over the whole share instead, every
 // CTA read the query fragments, and a power-of-two spacing put all the pages on the CTAs of one XCD (us a
 // launch, 32 heads, 131,072-token tables, requests x 6 rows: 1 of 2048 / 8192 / 32,768 tokens 7.3 / 8.1 /
-// 8.3 -> 5.0 / 4.9 / 6.1, 4 of 2048 / 8192 7.1 / 7.8 -> 5.2 / 6.2; 64 heads, 1 x 8 rows of 2048 8.8 -> 6.6).
+// 8.3 -> 5.0 / 4.8 / 6.1, 4 of 2048 / 8192 7.1 / 7.8 -> 5.1 / 6.3; 64 heads, 1 x 8 rows of 2048 8.8 -> 6.6).
 constexpr int kZeroCtas = 16;
 __device__ __forceinline__ int group_ctas(int pages, int total_pages, int target) {
   if (pages == 0) return 1;
@@ -181,6 +183,7 @@ __device__ void assign_cta(const DecodeArgs& a, int (&s_w)[2][NT / kWave], int* 
       my_pages += gp[i];
     }
   } else {
+#pragma unroll 1
     for (int g = g_lo; g < g_hi; ++g) my_pages += group_pages<R>(a, g);
   }
   int total_pages;
@@ -191,11 +194,13 @@ __device__ void assign_cta(const DecodeArgs& a, int (&s_w)[2][NT / kWave], int* 
 #pragma unroll
     for (int i = 0; i < kGpt; ++i) my_ctas += g_lo + i < g_hi ? group_ctas(gp[i], total_pages, a.target) : 0;
   } else {
+#pragma unroll 1
     for (int g = g_lo; g < g_hi; ++g) my_ctas += group_ctas(group_pages<R>(a, g), total_pages, a.target);
   }
   int total_ctas;
   int c0 = block_excl_sum<NT>(my_ctas, total_ctas, s_w[1]);
   if (cta >= c0 && cta < c0 + my_ctas) {
+#pragma unroll 1
     for (int i = 0; g_lo + i < g_hi; ++i) {
       int p;
       if (cached) {
@@ -376,42 +381,11 @@ __global__ __launch_bounds__((Shape<H, R, kHist>::kThreads)) __attribute__((amdg
     p_begin = jc * a.slice_pages;
     p_end = min(p_begin + a.slice_pages, pages);
     if (p_begin >= p_end) return;  // no page of this group in the slice
-  } else if (pages < nj) {  // block-uniform: a page each for the group's first CTAs
-    p_begin = min(jc, pages);
-    p_end = min(jc + 1, pages);
   } else {
     p_begin = static_cast<int>(static_cast<int64_t>(pages) * jc / nj);
     p_end = static_cast<int>(static_cast<int64_t>(pages) * (jc + 1) / nj);
   }
   const int n_local = p_end - p_begin;  // <= Sh::kMaxPages by the host's choice of target
-  // Mask words of the group's rows past its pages (no CTA scores them) are zeroed by the
-  // group's CTAs, a share each: one 8-B store per page and row when the layout allows it.
-  // Issued after the page stream, so that no DMA wait covers these stores.
-  auto zero_mask_tail = [&]() {
-    const int tail = a.bt_pages - pages;
-    const int units = R * tail;
-    const int u0 = static_cast<int>(static_cast<int64_t>(units) * jc / nj);
-    const int u1 = static_cast<int>(static_cast<int64_t>(units) * (jc + 1) / nj);
-    const bool wide = (reinterpret_cast<uintptr_t>(a.mask) & 7u) == 0 && (a.mask_stride & 3) == 0;
-    for (int u = kMask && a.mask != nullptr ? u0 + tid : u1; u < u1; u += NT) {
-      const int rr = u / tail;
-      int16_t* m = a.mask + static_cast<int64_t>(row0 + rr) * a.mask_stride + (pages + u - rr * tail) * 4;
-      if (wide) {
-        *reinterpret_cast<uint64_t*>(m) = 0;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m[e] = 0;
-      }
-    }
-  };
-  // A CTA without a page (kZeroCtas) only zeroes its share.
-  if constexpr (!kHist) {
-    if (n_local == 0) {  // block-uniform
-      zero_mask_tail();
-      zero_share();
-      return;
-    }
-  }
   // the pages this wave scores: without a mask to write, those that hold tokens of its row
   const int n_mine = kMask ? n_local : min(n_local, (len + kPage - 1) / kPage - p_begin);
   const int32_t* btr = a.bt + static_cast<int64_t>(group_row) * a.bt_stride + p_begin;
@@ -453,6 +427,27 @@ __global__ __launch_bounds__((Shape<H, R, kHist>::kThreads)) __attribute__((amdg
     for (int i = tid; i < R * kBins / 2; i += NT) s_hist[i] = 0;
     if (tid < 2 * R) s_cnt[tid] = 0;
   }
+  // Mask words of the group's rows past its pages (no CTA scores them) are zeroed by the
+  // group's CTAs, a share each: one 8-B store per page and row when the layout allows it.
+  // Issued after the page stream, so that no DMA wait covers these stores.
+  auto zero_mask_tail = [&]() {
+    const int tail = a.bt_pages - pages;
+    const int units = R * tail;
+    const int u0 = static_cast<int>(static_cast<int64_t>(units) * jc / nj);
+    const int u1 = static_cast<int>(static_cast<int64_t>(units) * (jc + 1) / nj);
+    const bool wide = (reinterpret_cast<uintptr_t>(a.mask) & 7u) == 0 && (a.mask_stride & 3) == 0;
+    for (int u = kMask && a.mask != nullptr ? u0 + tid : u1; u < u1; u += NT) {
+      const int rr = u / tail;
+      int16_t* m = a.mask + static_cast<int64_t>(row0 + rr) * a.mask_stride + (pages + u - rr * tail) * 4;
+      if (wide) {
+        *reinterpret_cast<uint64_t*>(m) = 0;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m[e] = 0;
+      }
+    }
+  };
+
   int nz = 0, pos = 0;
   const int n_steps = (n_local + S - 1) / S;  // block-uniform
   const int t_lo = lane & 15;
