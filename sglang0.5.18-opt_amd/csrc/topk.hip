@@ -1282,11 +1282,7 @@ __device__ __forceinline__ bool resolve_cands(ResolveLds<NT, CAP>& L, int n, con
 // path in one or two rounds), the row's quantile if its scores were normal (mean and deviation come
 // with the first count), a step from there by the normal density, then interpolation of the counts
 // between the bracket's float values with the Illinois weights; four or five rounds on the indexer's
-// logits.  A first count within a sixteenth of the row of 2048 takes the quantile's place, the step going
-// from zero (250 normal rows of 4096 tokens, six rounds -> four: 10.8 -> 9.9 us).  A round is about 0.65 us,
-// so rows far from normal, which take eight to twelve, gain nothing from being held where few rows are in
-// flight (64 rows of 2049-4096 tokens whose scores are ratios of normals 14.4 -> 16.2 us, 1024 x 4096 34 ->
-// 23).  Every third round from the sixth pulls the bracket's ends in to keys of the row, which ends
+// logits.  Every third round from the sixth pulls the bracket's ends in to keys of the row, which ends
 // the search on heavy ties, and past kHeldGuess rounds the probes halve the key range, so that no input
 // takes more than 32 further ones.
 constexpr int kHeldGuess = 18;
@@ -1460,19 +1456,10 @@ __device__ __forceinline__ void held_row(HeldLds<NT, Q>& L, const RowSrc& r, con
     const float mean = sum * inv_n;
     const float dev = __builtin_amdgcn_sqrtf(fmaxf(sq * inv_n - mean * mean, 0.0f));
     const float z = normal_quantile(static_cast<float>(kTopK) * inv_n);
-    const float per_key = 2.5066283f * dev * inv_n * __expf(0.5f * z * z);  // value a key there
     float next = mean + z * dev;  // the next probe's value, for the first two rounds
-    // a step past the 2048th from a probe that counted `off` keys too many, so that the two bracket it
-    auto step = [&](float from, int off) {
-      return from + (static_cast<float>(off) * 1.2f + (off >= 0 ? 20.0f : -20.0f)) * per_key;
-    };
     int side = 0;
     bool at_zero = n_pos < kTopK;  // first +0 itself: with its ties it may hold the 2048th
     int round = 0;
-    if (16 * abs(n_pos - kTopK) < len) {  // zero was as good a probe as the quantile will be
-      next = step(0.0f, n_pos - kTopK);
-      round = 1;
-    }
     while (lo < hi && c_lo - c_hi > kWave) {
       uint32_t p;  // a probe in (lo, hi]
       if (at_zero) {
@@ -1503,7 +1490,11 @@ __device__ __forceinline__ void held_row(HeldLds<NT, Q>& L, const RowSrc& r, con
       }
       p = static_cast<uint32_t>(uniform(static_cast<int>(p)));
       const int c = count_ge(p);
-      if (!at_zero && round == 1) next = step(key_value(p), c - kTopK);
+      // a step past the quantile by the normal density there, so that the two probes bracket it
+      if (!at_zero && round == 1) {
+        const float off = static_cast<float>(c - kTopK) * 1.2f + (c >= kTopK ? 20.0f : -20.0f);
+        next = key_value(p) + off * 2.5066283f * dev * inv_n * __expf(0.5f * z * z);
+      }
       at_zero = false;
       if (c >= kTopK) {
         lo = p;
