@@ -168,11 +168,12 @@ __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirs
 
 // Block-wide (NT threads) exclusive prefix (thread order) and total of a per-thread count; one
 // barrier; s_w (NT / 64 words) must not be reused before the next barrier.
-template <int NT>
+template <int NT, bool kLaneId = false>
 __device__ __forceinline__ int block_excl_sum(int x, int& total, int* s_w) {
+  const int lane = kLaneId ? lane_id() : static_cast<int>(threadIdx.x & 63);
   const int w = threadIdx.x >> 6;
   const int inc = wave_prefix_sum(x);
-  if (lane_id() == kWave - 1) s_w[w] = inc;
+  if (lane == 63) s_w[w] = inc;
   __syncthreads();
   int before = 0, tot = 0;
 #pragma unroll

@@ -914,7 +914,8 @@ __device__ __forceinline__ void emit_row(const RowSrc& r, uint32_t thr, int rema
 constexpr int kEmitWords = kBins / 2;
 constexpr int kEmitWin = kEmitWords * 32;
 
-template <int NT, typename Each>
+// kLaneId: the lane index computed anew instead of kept since the row's start, a register less there.
+template <int NT, bool kLaneId = false, typename Each>
 __device__ __forceinline__ void emit_held(Each each, const int* n_ties, uint32_t* bits, uint16_t* pre, int* s_w,
                                           int len, int32_t* dst) {
   constexpr int WPT = kBins / NT;  // words a thread zeroes and counts; all of one part
@@ -950,7 +951,7 @@ __device__ __forceinline__ void emit_held(Each each, const int* n_ties, uint32_t
       c += __popc(q.w);
     }
     int total;
-    int ex = block_excl_sum<NT>(c, total, s_w);
+    int ex = block_excl_sum<NT, kLaneId>(c, total, s_w);
     int tot_a = 0;  // the first part's count in this window: the words of threads [0, NT / 2)
 #pragma unroll
     for (int v = 0; v < NT / kWave / 2; ++v) tot_a += s_w[v];
@@ -1262,7 +1263,7 @@ __device__ __forceinline__ bool resolve_cands(ResolveLds<NT, CAP>& L, int n, con
     }
     wave_slot(tie, &L.misc[3]);  // the tie count, read by emit_held after its first barrier
   }
-  emit_held<NT>(
+  emit_held<NT, !kVec && CAP == kCapS>(
       [&](auto&& fn) {
 #pragma unroll
         for (int j = 0; j < EPT; ++j)
@@ -1282,7 +1283,10 @@ __device__ __forceinline__ bool resolve_cands(ResolveLds<NT, CAP>& L, int n, con
 // path in one or two rounds), the row's quantile if its scores were normal (mean and deviation come
 // with the first count), a step from there by the normal density, then interpolation of the counts
 // between the bracket's float values with the Illinois weights; four or five rounds on the indexer's
-// logits.  Every third round from the sixth pulls the bracket's ends in to keys of the row, which ends
+// logits.  A round is about 0.65 us, so rows whose scores are far from normal, which take eight to twelve, gain
+// nothing from being held where few rows are in flight (64 rows of 2049-4096 tokens, ratios of normals 14.4 ->
+// 16.6 us; 1024 x 4096 34 -> 23), nor do 4096 normal scores, whose 2048th lies beside zero, the first count's own
+// probe (250 rows 9.4 -> 10.8).  Every third round from the sixth pulls the bracket's ends in to keys of the row, which ends
 // the search on heavy ties, and past kHeldGuess rounds the probes halve the key range, so that no input
 // takes more than 32 further ones.
 constexpr int kHeldGuess = 18;
